@@ -129,7 +129,7 @@ struct gla_opr_s {
     std::shared_ptr<std::vector<char>> fur_host;   // reference layout, operator dtype
     void* w1 = nullptr;
     void* w2 = nullptr;
-    int64_t ws_nrhs = 0;
+    int64_t w1_slots = 0, w2_slots = 0;   // right-hand sides (times partitions) w1 / w2 hold
     int batches = 0;   // recorded batches that use w1 / w2 (they must not move)
     // device copies of the host arrays of gla_opr_apply_host (grown as
     // needed, kept until release), under their own lock
@@ -446,14 +446,41 @@ void part_offset(int64_t p, const int64_t div[3], int o[3])
 
 size_t elem_bytes(int dtype) { return dtype == GLA_C64 ? 8 : 16; }
 
-// The whole matvec on `st` with work planes w1 / w2.  A partitioned operator
-// runs the five passes once per (source, target) partition pair: pass 1
-// gathers source partition s (genPrt), pass 5 writes or accumulates into
-// target partition t (mrgPrt); the first source partition of a target
-// partition applies (alpha, beta), the later ones add with beta = 1, which
-// is the leaf sum of egoBrnHst! (src/glaAct.jl:158-164) carried through the
-// inverse transforms (they are linear).
-hipError_t matvec_all(const gla_opr_s& h, const void* x, void* y, void* w1, void* w2, int nrhs, double ar,
+// Work-plane slots of nrhs right-hand sides.  A partitioned operator takes all
+// partitions of a pass in one launch (run_matvec_parts: each source partition
+// transformed once, the sum over them between the transforms) when its slots
+// stay within kPartBytes; otherwise, or when only that much work memory is at
+// hand, it runs the five passes once per (source, target) pair on one slot
+// per right-hand side.  48^3 fine cells (8 source partitions) on 24^3 coarse
+// ones, ComplexF32: 211 us pair by pair (40 launches of too few workgroups
+// each, the forward and inverse transforms of pass 3 once per pair), 69 us in
+// five launches.  The bound is on memory: it keeps the work planes of one
+// call within a hundredth of the GPU's.
+constexpr int64_t kPartBytes = (int64_t)2 << 30;
+
+struct Slots {
+    int64_t w1, w2;
+};
+
+Slots pair_slots(int64_t nrhs) { return Slots{nrhs, nrhs}; }
+
+Slots part_slots(const gla_opr_s& h, int64_t nrhs)
+{
+    const int64_t Ps = n_src_part(h.dims), Pt = n_trg_part(h.dims);
+    if (Ps * Pt == 1) return pair_slots(nrhs);
+    const Slots s{nrhs * std::max(Ps, Pt), nrhs * (Ps + (Pt > 1 ? Pt : 0))};
+    const int64_t bytes = (s.w1 * h.geom.w1s + s.w2 * h.geom.w2s) * (int64_t)elem_bytes(h.dims.dtype);
+    return s.w1 <= 65535 && bytes <= kPartBytes ? s : pair_slots(nrhs);
+}
+
+// The whole matvec on `st` with work planes w1 / w2 of `have` slots.  Pair by
+// pair, a partitioned operator's pass 1 gathers source partition s (genPrt)
+// and pass 5 writes or accumulates into target partition t (mrgPrt); the
+// first source partition of a target partition applies (alpha, beta), the
+// later ones add with beta = 1, which is the leaf sum of egoBrnHst!
+// (src/glaAct.jl:158-164) carried through the inverse transforms (they are
+// linear).
+hipError_t matvec_all(const gla_opr_s& h, const void* x, void* y, void* w1, void* w2, Slots have, int nrhs, double ar,
                       double ai, double br, double bi, int axpby, const gla::Epi& epi, hipStream_t st)
 {
     const bool c64 = h.dims.dtype == GLA_C64;
@@ -464,11 +491,17 @@ hipError_t matvec_all(const gla_opr_s& h, const void* x, void* y, void* w1, void
     const int64_t Ps = n_src_part(h.dims), Pt = n_trg_part(h.dims);
     if (Ps * Pt == 1) return one(h.geom, h.tab, br, bi, axpby);
     if (axpby == 2) return hipErrorInvalidValue;   // self operators only, never partitioned
+    const int64_t pair = 8 * h.dims.fur_ext[0] * h.dims.fur_ext[1] * h.dims.fur_ext[2] * 6;
+    const Slots s = part_slots(h, nrhs);
+    if (s.w1 > nrhs && have.w1 >= s.w1 && have.w2 >= s.w2)
+        return c64 ? gla::run_matvec_parts<float>(h.geom, h.tab, x, y, w1, w2, nrhs, (int)Ps, (int)Pt, pair, ar, ai, br,
+                                                  bi, axpby, st)
+                   : gla::run_matvec_parts<double>(h.geom, h.tab, x, y, w1, w2, nrhs, (int)Ps, (int)Pt, pair, ar, ai,
+                                                   br, bi, axpby, st);
     if (axpby == 0) {
         ar = 1; ai = 0; br = 0; bi = 0;
     }
-    const int64_t blk = 8 * h.dims.fur_ext[0] * h.dims.fur_ext[1] * h.dims.fur_ext[2] * 6 *
-                        (int64_t)elem_bytes(h.dims.dtype);
+    const int64_t blk = pair * (int64_t)elem_bytes(h.dims.dtype);
     for (int64_t t = 0; t < Pt; ++t)
         for (int64_t s = 0; s < Ps; ++s) {
             gla::Geom g = h.geom;
@@ -482,19 +515,44 @@ hipError_t matvec_all(const gla_opr_s& h, const void* x, void* y, void* w1, void
     return hipSuccess;
 }
 
-gla_status ensure_ws(gla_opr_t h, int64_t nrhs)
+// Work buffers of nrhs right-hand sides (GLA_OK also when they cannot grow but
+// hold what the pair-by-pair form needs).
+gla_status ensure_ws(gla_opr_t h, int64_t nrhs, bool may_grow = true)
 {
-    if (h->ws_nrhs >= nrhs) return GLA_OK;
+    const Slots want = part_slots(*h, nrhs);
+    if (h->w1_slots >= want.w1 && h->w2_slots >= want.w2) return GLA_OK;
+    const bool fits = h->w1_slots >= nrhs && h->w2_slots >= nrhs;
+    if (fits && (!may_grow || h->batches > 0)) return GLA_OK;
+    if (!may_grow)
+        return fail(GLA_ERR_ARG, "work buffers for " + std::to_string(nrhs) +
+                                     " right-hand sides must be reserved (gla_opr_reserve) before capture");
     if (h->batches > 0)
         return fail(GLA_ERR_ARG, "the operator's work buffers are recorded in a batch; "
                                  "destroy the batch before applying it to more right-hand sides");
     const size_t eb = elem_bytes(h->dims.dtype);
     if (h->w1) { (void)hipFree(h->w1); h->w1 = nullptr; }
     if (h->w2) { (void)hipFree(h->w2); h->w2 = nullptr; }
-    h->ws_nrhs = 0;
-    GLA_HIP(hipMalloc(&h->w1, (size_t)(h->geom.w1s * nrhs) * eb));
-    GLA_HIP(hipMalloc(&h->w2, (size_t)(h->geom.w2s * nrhs) * eb));
-    h->ws_nrhs = nrhs;
+    h->w1_slots = h->w2_slots = 0;
+    auto grow = [&](Slots s) {
+        hipError_t e = hipMalloc(&h->w1, (size_t)(h->geom.w1s * s.w1) * eb);
+        if (e != hipSuccess) { h->w1 = nullptr; return e; }
+        e = hipMalloc(&h->w2, (size_t)(h->geom.w2s * s.w2) * eb);
+        if (e != hipSuccess) {
+            h->w2 = nullptr;
+            (void)hipFree(h->w1);
+            h->w1 = nullptr;
+            return e;
+        }
+        h->w1_slots = s.w1;
+        h->w2_slots = s.w2;
+        return e;
+    };
+    hipError_t e = grow(want);
+    if (e != hipSuccess && want.w1 > nrhs) {
+        (void)hipGetLastError();
+        e = grow(pair_slots(nrhs));
+    }
+    if (e != hipSuccess) return fail(GLA_ERR_HIP, std::string("hipMalloc of the work buffers: ") + hipGetErrorString(e));
     return GLA_OK;
 }
 
@@ -510,18 +568,16 @@ gla_status run(gla_opr_t h, const void* x, int64_t nx, void* y, int64_t ny, int6
     if (ny != h->geom.ys * nrhs) return fail(GLA_ERR_SIZE, "Size of output vector does not match the target volume.");
     std::lock_guard<std::mutex> lk(h->mu);
     DevGuard g(h->opts.device);
-    if (h->ws_nrhs < nrhs) {
-        // growing the work buffers frees and allocates, which a stream under
-        // graph capture must not see
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        if (stream && hipStreamIsCapturing((hipStream_t)stream, &cs) == hipSuccess &&
-            cs != hipStreamCaptureStatusNone)
-            return fail(GLA_ERR_ARG, "work buffers for " + std::to_string(nrhs) +
-                                         " right-hand sides must be reserved (gla_opr_reserve) before capture");
-    }
-    gla_status s = ensure_ws(h, nrhs);
+    // growing the work buffers frees and allocates, which a stream under
+    // graph capture must not see
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    const Slots want = part_slots(*h, nrhs);
+    const bool enough = h->w1_slots >= want.w1 && h->w2_slots >= want.w2;
+    const bool capturing = !enough && stream && hipStreamIsCapturing((hipStream_t)stream, &cs) == hipSuccess &&
+                           cs != hipStreamCaptureStatusNone;
+    gla_status s = ensure_ws(h, nrhs, !capturing);
     if (s) return s;
-    const hipError_t e = matvec_all(*h, x, y, h->w1, h->w2, (int)nrhs, ar, ai, br, bi, axpby, epi,
+    const hipError_t e = matvec_all(*h, x, y, h->w1, h->w2, Slots{h->w1_slots, h->w2_slots}, (int)nrhs, ar, ai, br, bi, axpby, epi,
                                     (hipStream_t)stream);
     if (e != hipSuccess) return fail(GLA_ERR_HIP, std::string("matvec launch: ") + hipGetErrorString(e));
     return GLA_OK;
@@ -879,9 +935,13 @@ gla_status gla_opr_apply_noalloc(gla_opr_t h, const void* x, int64_t nx, void* y
                                   "layout is (srcCelX, srcCelY, srcCelZ, 3).");
     if (ny != h->geom.ys * nrhs) return fail(GLA_ERR_SIZE, "Size of output vector does not match the target volume.");
     const size_t eb = elem_bytes(h->dims.dtype);
-    // W1 then W2, each start on a 256-byte boundary
-    const size_t w1b = ((size_t)(h->geom.w1s * nrhs) * eb + 255) & ~(size_t)255;
-    const size_t need = w1b + (size_t)(h->geom.w2s * nrhs) * eb;
+    // W1 then W2, each start on a 256-byte boundary; a partitioned operator
+    // whose partitions do not fit together runs pair by pair
+    auto bytes1 = [&](Slots s) { return ((size_t)(h->geom.w1s * s.w1) * eb + 255) & ~(size_t)255; };
+    auto bytes = [&](Slots s) { return bytes1(s) + (size_t)(h->geom.w2s * s.w2) * eb; };
+    Slots have = part_slots(*h, nrhs);
+    if (bytes(have) > kScratchBytes) have = pair_slots(nrhs);
+    const size_t w1b = bytes1(have), need = bytes(have);
     if (need > kScratchBytes)
         return fail(GLA_ERR_SIZE, "the allocation-free matvec needs " + std::to_string(need) +
                                       " bytes of work memory, more than its fixed " + std::to_string(kScratchBytes) +
@@ -893,7 +953,7 @@ gla_status gla_opr_apply_noalloc(gla_opr_t h, const void* x, int64_t nx, void* y
     DevGuard g(h->opts.device);
     void* w1 = base;
     void* w2 = (unsigned char*)base + w1b;
-    const hipError_t e = matvec_all(*h, x, y, w1, w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(), (hipStream_t)stream);
+    const hipError_t e = matvec_all(*h, x, y, w1, w2, have, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(), (hipStream_t)stream);
     if (e != hipSuccess) return fail(GLA_ERR_HIP, std::string("matvec launch: ") + hipGetErrorString(e));
     return GLA_OK;
 }
@@ -1178,7 +1238,7 @@ gla_status gla_batch_create(const gla_opr_t* ops, const void* const* x, void* co
         std::lock_guard<std::mutex> lk(h->mu);
         const int r = (int)(nrhs ? nrhs[i] : 1);
         hipStream_t st = ls[(size_t)lane[(size_t)i]];
-        e = matvec_all(*h, x[i], y[i], h->w1, h->w2, r, 1, 0, 0, 0, 0, gla::Epi(), st);
+        e = matvec_all(*h, x[i], y[i], h->w1, h->w2, Slots{h->w1_slots, h->w2_slots}, r, 1, 0, 0, 0, 0, gla::Epi(), st);
     }
     for (int k = 0; k < lanes && e == hipSuccess; ++k) e = hipEventRecord(ev[(size_t)k], ls[(size_t)k]);
     for (int k = 0; k < lanes && e == hipSuccess; ++k) e = hipStreamWaitEvent(cap, ev[(size_t)k], 0);   // join
@@ -1230,7 +1290,8 @@ gla_status gla_opr_reserve(gla_opr_t h, int64_t nrhs)
 int64_t gla_opr_workspace_bytes(gla_opr_t h, int64_t nrhs)
 {
     if (!h) return -1;
-    return (h->geom.w1s + h->geom.w2s) * nrhs * (int64_t)elem_bytes(h->dims.dtype);
+    const Slots s = part_slots(*h, nrhs);
+    return (h->geom.w1s * s.w1 + h->geom.w2s * s.w2) * (int64_t)elem_bytes(h->dims.dtype);
 }
 
 int64_t gla_krylov_dots_workspace(int64_t k, int64_t nv, int64_t n)

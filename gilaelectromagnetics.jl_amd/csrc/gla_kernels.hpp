@@ -43,10 +43,26 @@ constexpr int yk_of()
 // (target): cell (i1, i2, i3) of the partition is cell (i_d * d_d + o_d) of
 // the full volume of f_d cells per axis (genPrt / mrgPrt,
 // src/glaActSup.jl:4-18, 939-953).  Unpartitioned: f = the volume, d = 1,
-// o = 0.
+// o = 0.  A launch over np partitions of every right-hand side takes them in
+// the order of GlaExtInf (x fastest) from partition o on, slot rhs np + p
+// partition p of right-hand side rhs.
 struct Part {
-    int f[3], d[3], o[3];
+    int f[3], d[3], o[3], np;
 };
+
+// right-hand side and partition offset of a launch's slot
+__device__ __forceinline__ int part_slot(const Part& a, int slot, int (&o)[3])
+{
+    o[0] = a.o[0];
+    o[1] = a.o[1];
+    o[2] = a.o[2];
+    if (a.np == 1) return slot;
+    const int p = slot % a.np;
+    o[0] += p % a.d[0];
+    o[1] += p / a.d[0] % a.d[1];
+    o[2] += p / (a.d[0] * a.d[1]);
+    return slot / a.np;
+}
 
 
 // (i2, i3, c) of row `pen` of a workgroup whose first row is `row0`, rows
@@ -218,9 +234,11 @@ __global__ __launch_bounds__(TP * PEN, MINW) void k_fwd_x(const cpx<R>* __restri
     row_coords(blockIdx.x * PEN, act ? pen : 0, S2, S3, i2, i3, c);
     // the row of source partition xp (the whole volume's row without
     // partitions: xp.f = S, xp.d = 1, xp.o = 0)
-    const cpx<R>* xr = X + (int64_t)blockIdx.y * xs +
-                       ((((int64_t)c * xp.f[2] + (int64_t)i3 * xp.d[2] + xp.o[2]) * xp.f[1] + (int64_t)i2 * xp.d[1] +
-                         xp.o[1]) * xp.f[0] + xp.o[0]);
+    int po[3];
+    const int rhs = part_slot(xp, blockIdx.y, po);
+    const cpx<R>* xr = X + (int64_t)rhs * xs +
+                       ((((int64_t)c * xp.f[2] + (int64_t)i3 * xp.d[2] + po[2]) * xp.f[1] + (int64_t)i2 * xp.d[1] +
+                         po[1]) * xp.f[0] + po[0]);
     const int xd = xp.d[0];
     cpx<R>* wr = W1 + (int64_t)blockIdx.y * ws + (((int64_t)c * Z + i3) * Y1 + i2) * (2 * N);
     cpx<R> v[2][E];   // even, odd parity
@@ -285,9 +303,11 @@ __global__ __launch_bounds__(TP * PEN, MINW) void k_inv_x(const cpx<R>* __restri
     // the row of target partition yp (the whole volume's row without
     // partitions); the Lippmann-Schwinger form (axpby 2) is for self
     // operators, never partitioned
-    cpx<R>* yr = Y + (int64_t)blockIdx.y * ys +
-                 ((((int64_t)c * yp.f[2] + (int64_t)i3 * yp.d[2] + yp.o[2]) * yp.f[1] + (int64_t)i2 * yp.d[1] + yp.o[1]) *
-                      yp.f[0] + yp.o[0]);
+    int po[3];
+    const int rhs = part_slot(yp, blockIdx.y, po);
+    cpx<R>* yr = Y + (int64_t)rhs * ys +
+                 ((((int64_t)c * yp.f[2] + (int64_t)i3 * yp.d[2] + po[2]) * yp.f[1] + (int64_t)i2 * yp.d[1] + po[1]) *
+                      yp.f[0] + po[0]);
     const int yd = yp.d[0];
     const int64_t cell0 = ((int64_t)i3 * T2 + i2) * T1;
     cpx<R> v[2][E];
@@ -726,6 +746,163 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_zpass(cpx<R>* __restrict__ W2
             if (n < top) *cp(c, TP * e) = acc[c][e];
             if constexpr (MODE == 2)
                 if (n + N < T3) *cp(c, TP * e + N) = accb[c][e];
+        }
+}
+
+// --------------------------------------------------------------------------
+// Pass 3 of a partitioned operator: for target partition tp,
+//   Wo[tp] = IDFT_3( sum_s G^_{s,tp} DFT_3(W2[s]) ),
+// the sum over the Ps source partitions taken between the transforms (the
+// leaf sum of egoBrnHst!, src/glaAct.jl:158-164), so every partition is
+// transformed once forward per target partition and the result once back.
+// blockDim / (TP PX) thread groups share the source partitions of a tile and
+// add their sums through LDS; group 0 transforms back and stores.  Bound by
+// latency at the sizes partitions have (48^3 fine cells on 24^3, ComplexF32:
+// 288 tiles): the groups shorten the chain of transforms of one tile from Ps
+// to Ps / groups.
+// With Pt == 1 Wo may be W2's first slot (a workgroup owns its columns in
+// every slot: its stores follow all its loads).
+// Workspace slots: W2 rhs Ps + s, Wo as given by the stride ws of slot
+// rhs Pt + tp.  G^ block of a pair: (s + Ps tp) gpair entries on.
+// --------------------------------------------------------------------------
+template <typename R, int N, int TP, int PX, int MODE, int KB>
+__global__ __launch_bounds__(TP * PX > 512 ? TP * PX : 512) void k_zpart(
+    const cpx<R>* W2, cpx<R>* Wo, int L1, int L2, int S3, int T3, int Z, int64_t w2s, int64_t wos,
+    const cpx<R>* __restrict__ gf, int64_t gpair, AxisMap a1, AxisMap a2, AxisMap a3, const cpx<R>* __restrict__ phz,
+    const cpx<R>* __restrict__ tw, const int* __restrict__ order, int per_xcd, int nrhs, int Ps, int Pt)
+{
+    constexpr int E = N / TP, NT = TP * PX;
+    extern __shared__ __align__(16) unsigned char smem[];
+    cpx<R>* const tab = reinterpret_cast<cpx<R>*>(smem);
+    const int sg = threadIdx.x / NT, ng = blockDim.x / NT, lt = threadIdx.x % NT;
+    cpx<R>* const buf = tab + 2 * N;
+    cpx<R>* const lds = buf + sg * (KB * PX * N);
+    const int xl = lt % PX, t = lt / PX;
+    using FftF3 = PencilFft<R, N, TP, PX, 1, false, 0, 3, PX * N>;
+    using FftI3 = PencilFft<R, N, TP, PX, 1, true, 0, 3, PX * N>;
+    using FftF1 = PencilFft<R, N, TP, PX, 1, false>;
+    using FftI1 = PencilFft<R, N, TP, PX, 1, true>;
+    // workgroup -> (tile, target partition, right-hand side): all right-hand
+    // sides of a tile and target partition follow one another on one XCD
+    const int per = nrhs * Pt;
+    const int q = blockIdx.x / 8;
+    const int tile = order[(blockIdx.x % 8) * per_xcd + q / per];
+    if (tile < 0) return;   // padding entry (whole workgroup)
+    const int tp = q % per / nrhs, rhs = q % nrhs;
+    const int m1 = (tile & 0xffff) * PX + xl, m2 = tile >> 16;
+    const bool act = m1 < L1;
+    for (int i = threadIdx.x; i < N; i += blockDim.x) {
+        tab[i] = tw[i];
+        tab[N + i] = phz[i];
+    }
+    __syncthreads();
+    const int64_t cs = (int64_t)Z * L2 * L1, zs = (int64_t)L2 * L1;
+    const int64_t col = (int64_t)m2 * L1 + m1 + (int64_t)t * zs;
+    const int p1 = act && m1 >= a1.B ? 1 : 0, k1 = act ? m1 - p1 * a1.B : 0;
+    const int p2 = m2 >= a2.B ? 1 : 0, k2 = m2 - p2 * a2.B;
+    int j1, s1, j2, s2;
+    axis_lookup(a1, p1, k1, j1, s1);
+    axis_lookup(a2, p2, k2, j2, s2);
+    const int uu = a1.U * a2.U;
+    cpx<R> acc[3][E];
+    cpx<R> accb[MODE == 2 ? 3 : 1][MODE == 2 ? E : 1];
+#pragma unroll
+    for (int p3 = 0; p3 < 2; ++p3) {
+        cpx<R> sum[3][E];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int e = 0; e < E; ++e) sum[c][e] = {R(0), R(0)};
+        const cpx<R>* const gcol =
+            gf + (int64_t)Ps * tp * gpair +
+            ((int64_t)((p1 << 2) | (p2 << 1) | p3) * a3.U * uu + (int64_t)(j2 * a1.U + j1)) * 6;
+        for (int s0 = 0; s0 < Ps; s0 += ng) {
+            const int s = s0 + sg;
+            const bool on = act && s < Ps;
+            const cpx<R>* const x = W2 + ((int64_t)rhs * Ps + s) * w2s + col;
+            cpx<R> w[3][E];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    const int n = t + TP * e;
+                    const cpx<R> a = on && n < S3 ? x[c * cs + (int64_t)(TP * e) * zs] : cpx<R>{R(0), R(0)};
+                    if constexpr (MODE == 1) {
+                        const cpx<R> b = on && n + N < S3 ? x[c * cs + (int64_t)(TP * e + N) * zs] : cpx<R>{R(0), R(0)};
+                        w[c][e] = p3 == 0 ? a + b : tab[N + n] * (a - b);
+                    } else {
+                        w[c][e] = p3 == 0 ? a : tab[N + n] * a;
+                    }
+                }
+            if constexpr (KB == 3) {
+                FftF3::run(w, lds, t, xl, tab);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) FftF1::run(w[c], lds, t, xl, tab);
+            }
+            if (on) {
+                const cpx<R>* const gb = gcol + (int64_t)s * gpair;
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    int j3, s3;
+                    axis_lookup(a3, p3, t + TP * e, j3, s3);
+                    const cpx<R>* const g = gb + (int64_t)(j3 * uu) * 6;
+                    const cpx<R> gxx = g[0], gyy = g[1], gzz = g[2];
+                    const cpx<R> gxy = R(s1 * s2) * g[3], gxz = R(s1 * s3) * g[4], gyz = R(s2 * s3) * g[5];
+                    const cpx<R> x0 = w[0][e], x1 = w[1][e], x2 = w[2][e];
+                    sum[0][e] = sum[0][e] + (gxx * x0 + gxy * x1 + gxz * x2);
+                    sum[1][e] = sum[1][e] + (gxy * x0 + gyy * x1 + gyz * x2);
+                    sum[2][e] = sum[2][e] + (gxz * x0 + gyz * x1 + gzz * x2);
+                }
+            }
+        }
+        // the groups' sums, in their order, to group 0 (the buffers are free:
+        // a transform ends with a barrier)
+        if (ng > 1) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+#pragma unroll
+                for (int e = 0; e < E; ++e) lds[e * NT + lt] = sum[c][e];
+                __syncthreads();
+                if (sg == 0)
+                    for (int o = 1; o < ng; ++o)
+#pragma unroll
+                        for (int e = 0; e < E; ++e)
+                            sum[c][e] = sum[c][e] + buf[o * (KB * PX * N) + e * NT + lt];
+                __syncthreads();
+            }
+        }
+        if constexpr (KB == 3) {
+            FftI3::run(sum, lds, t, xl, tab);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) FftI1::run(sum[c], lds, t, xl, tab);
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if (p3 == 0) {
+                    acc[c][e] = sum[c][e];
+                    if constexpr (MODE == 2) accb[c][e] = sum[c][e];
+                } else {
+                    const cpx<R> po = cmulc(sum[c][e], tab[N + t + TP * e]);
+                    acc[c][e] = acc[c][e] + po;
+                    if constexpr (MODE == 2) accb[c][e] = accb[c][e] - po;
+                }
+            }
+    }
+    if (!act || sg != 0) return;
+    cpx<R>* const y = Wo + ((int64_t)rhs * Pt + tp) * wos + col;
+    const int top = T3 < N ? T3 : N;
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int n = t + TP * e;
+            if (n < top) y[c * cs + (int64_t)(TP * e) * zs] = acc[c][e];
+            if constexpr (MODE == 2)
+                if (n + N < T3) y[c * cs + (int64_t)(TP * e + N) * zs] = accb[c][e];
         }
 }
 

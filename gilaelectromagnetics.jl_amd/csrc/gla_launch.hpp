@@ -32,6 +32,7 @@ inline Part whole_part(const int* n)
 {
     Part p{};
     for (int a = 0; a < 3; ++a) { p.f[a] = n[a]; p.d[a] = 1; p.o[a] = 0; }
+    p.np = 1;
     return p;
 }
 
@@ -86,5 +87,14 @@ template <typename R>
 hipError_t run_matvec(const Geom& g, const DevTab& tb, const void* X, void* Y, void* W1, void* W2,
                       int nrhs, double ar, double ai, double br, double bi, int axpby, const Epi& epi,
                       hipStream_t st);
+
+// A partitioned operator's matvec with all partitions of a pass in one launch
+// (Ps source, Pt target partitions, gpair G^ entries per pair): work planes
+// of nrhs max(Ps, Pt) slots (W1) and nrhs Ps slots, for Pt > 1 followed by
+// nrhs Pt more (W2)
+template <typename R>
+hipError_t run_matvec_parts(const Geom& g, const DevTab& tb, const void* X, void* Y, void* W1, void* W2, int nrhs,
+                            int Ps, int Pt, int64_t gpair, double ar, double ai, double br, double bi, int axpby,
+                            hipStream_t st);
 
 }  // namespace gla

@@ -132,7 +132,7 @@ static hipError_t launch_fwd_x(const Geom& g, const DevTab& tb, const void* X, v
 {
     using K = LenK<R, N>;
     const int rows = g.S[1] * g.S[2] * 3;
-    dim3 grid((rows + K::PEN - 1) / K::PEN, nrhs);
+    dim3 grid((rows + K::PEN - 1) / K::PEN, nrhs * g.xp.np);
     hipLaunchKernelGGL((k_fwd_x<R, N, K::TP_ROW, K::PEN, 1>), grid, dim3(K::TP_ROW * K::PEN), 0, st,
                        (const cpx<R>*)X, (cpx<R>*)W1, g.S[0], g.S[1], g.S[2], g.Y1, g.Z, g.xs, g.w1s,
                        (const cpx<R>*)tb.phz[0], (const cpx<R>*)tb.tw[0], g.xp);
@@ -145,7 +145,7 @@ static hipError_t launch_inv_x(const Geom& g, const DevTab& tb, const void* W1, 
 {
     using K = LenK<R, N>;
     const int rows = g.T[1] * g.T[2] * 3;
-    dim3 grid((rows + K::PEN - 1) / K::PEN, nrhs);
+    dim3 grid((rows + K::PEN - 1) / K::PEN, nrhs * g.yp.np);
     hipLaunchKernelGGL((k_inv_x<R, N, K::TP_ROW, K::PEN, 1>), grid, dim3(K::TP_ROW * K::PEN), 0, st,
                        (const cpx<R>*)W1, (cpx<R>*)Y, g.T[0], g.T[1], g.T[2], g.Y1, g.Z, g.w1s, g.ys,
                        (const cpx<R>*)tb.phz[0], (const cpx<R>*)tb.tw[0], al, be, axpby,
@@ -284,6 +284,71 @@ hipError_t run_matvec(const Geom& g, const DevTab& tb, const void* X, void* Y, v
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
+}
+
+// pass 3 of a partitioned operator on the shape of pass 3; the thread groups
+// of a workgroup take the source partitions side by side within 512 threads
+// and GLA_ZBATCH_KB of exchange buffers
+template <typename R, int N, int SMALL>
+static hipError_t launch_zpart_shape(const Geom& g, const DevTab& tb, void* W2, void* Wo, int64_t wos, int nrhs,
+                                     int Ps, int Pt, int64_t gpair, hipStream_t st)
+{
+    using K = ZK<R, N, SMALL>;
+    constexpr int NT = K::TP_Z * K::PXZ, BUF = K::KB_Z * K::PXZ * N * (int)sizeof(cpx<R>);
+    int ng = 1;
+    while (2 * ng <= Ps && 2 * ng * NT <= 512 && 2 * ng * BUF <= GLA_ZBATCH_KB * 1024) ng *= 2;
+    const int64_t wgs = 8LL * tb.zper_xcd * nrhs * Pt;
+    if (wgs > 2147483647LL) return hipErrorInvalidValue;
+    const size_t lds = (size_t)ng * BUF + 2 * N * sizeof(cpx<R>);
+    auto go = [&](auto kernel) {
+        if (lds > 65536) {
+            const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     (int)lds);
+            if (e != hipSuccess) return e;
+        }
+        hipLaunchKernelGGL(kernel, dim3((unsigned)wgs), dim3(NT * ng), lds, st, (const cpx<R>*)W2, (cpx<R>*)Wo,
+                           g.L[0], g.L[1], g.S[2], g.T[2], g.Z, g.w2s, wos, (const cpx<R>*)tb.gf, gpair, tb.am[0],
+                           tb.am[1], tb.am[2], (const cpx<R>*)tb.phz[2], (const cpx<R>*)tb.tw[2], tb.zorder,
+                           tb.zper_xcd, nrhs, Ps, Pt);
+        return hipGetLastError();
+    };
+    if (g.S[2] > g.B[2]) return go(k_zpart<R, N, K::TP_Z, K::PXZ, 1, K::KB_Z>);
+    if (g.T[2] > g.B[2]) return go(k_zpart<R, N, K::TP_Z, K::PXZ, 2, K::KB_Z>);
+    return go(k_zpart<R, N, K::TP_Z, K::PXZ, 0, K::KB_Z>);
+}
+
+template <typename R, int N>
+static hipError_t launch_zpart(const Geom& g, const DevTab& tb, void* W2, void* Wo, int64_t wos, int nrhs, int Ps,
+                               int Pt, int64_t gpair, hipStream_t st)
+{
+    return (int64_t)g.L[0] * g.L[1] < ZSMALL_COLS
+               ? launch_zpart_shape<R, N, 1>(g, tb, W2, Wo, wos, nrhs, Ps, Pt, gpair, st)
+               : launch_zpart_shape<R, N, 0>(g, tb, W2, Wo, wos, nrhs, Ps, Pt, gpair, st);
+}
+
+template <typename R>
+hipError_t run_matvec_parts(const Geom& g0, const DevTab& tb, const void* X, void* Y, void* W1, void* W2, int nrhs,
+                            int Ps, int Pt, int64_t gpair, double ar, double ai, double br, double bi, int axpby,
+                            hipStream_t st)
+{
+    Geom g = g0;
+    g.xp.np = Ps;
+    g.yp.np = Pt;
+    // pass 4 reads pass 3's results: in place of every right-hand side's
+    // first source slot, or in the slots behind
+    Geom go = g;
+    void* Wo = W2;
+    if (Pt == 1) go.w2s = (int64_t)Ps * g.w2s;
+    else Wo = (cpx<R>*)W2 + (int64_t)nrhs * Ps * g.w2s;
+    hipError_t e = run_pass<R>(0, g, tb, X, Y, W1, W2, nrhs, ar, ai, br, bi, axpby, Epi(), st);
+    if (e == hipSuccess) e = run_pass<R>(1, g, tb, X, Y, W1, W2, nrhs * Ps, ar, ai, br, bi, axpby, Epi(), st);
+    if (e != hipSuccess) return e;
+#define GLA_CASE_3(n) case n: e = launch_zpart<R, n>(g, tb, W2, Wo, go.w2s, nrhs, Ps, Pt, gpair, st); break;
+    switch (g.B[2]) { GLA_FOR_EACH_LEN(GLA_CASE_3) default: return hipErrorInvalidValue; }
+#undef GLA_CASE_3
+    if (e == hipSuccess) e = run_pass<R>(3, go, tb, X, Y, W1, Wo, nrhs * Pt, ar, ai, br, bi, axpby, Epi(), st);
+    if (e == hipSuccess) e = run_pass<R>(4, g, tb, X, Y, W1, W2, nrhs, ar, ai, br, bi, axpby, Epi(), st);
+    return e;
 }
 
 }  // namespace gla
