@@ -336,26 +336,88 @@ gla_status gla_opr_get_dims(gla_opr_t h, gla_dims* out)
 
 namespace {
 
+// Stored extent and mirror storage of an axis of the device G^.
+struct AxisStore {
+    int U;
+    bool sym;
+};
+
+// Whether the branches are their own mirror images along axis a up to
+// rounding, F(L - m) = s F(m) with s = -1 for the off-diagonal components
+// that involve the axis (the relation of a self axis).
+bool mirrored(const gla_dims& d, const std::vector<std::complex<double>>& fur, int a, double tol)
+{
+    const int64_t U[3] = {d.fur_ext[0], d.fur_ext[1], d.fur_ext[2]};
+    const int64_t Ut = U[0] * U[1] * U[2], B = U[a];
+    const int64_t st = a == 0 ? 1 : a == 1 ? U[0] : U[0] * U[1];
+    double top = 0;
+    for (const auto& v : fur) top = std::max(top, std::max(std::fabs(v.real()), std::fabs(v.imag())));
+    const double lim = tol * top;
+    static const int odd[3][2] = {{3, 4}, {3, 5}, {4, 5}};
+    for (int b = 0; b < 8; ++b)
+        for (int c = 0; c < 6; ++c) {
+            const std::complex<double>* const f = &fur[(size_t)((b * 6 + c) * Ut)];
+            const double s = (c == odd[a][0] || c == odd[a][1]) ? -1.0 : 1.0;
+            const int p = (b >> (2 - a)) & 1;
+            for (int64_t lo = 0; lo < Ut; lo += st * B)
+                for (int64_t k = 0; 2 * k <= B; ++k) {
+                    const int64_t m = p ? B - 1 - k : (B - k) % B;
+                    const std::complex<double>*const u = f + lo + k * st, *const v = f + lo + m * st;
+                    for (int64_t i = 0; i < st; ++i)
+                        if (std::fabs(v[i].real() - s * u[i].real()) > lim ||
+                            std::fabs(v[i].imag() - s * u[i].imag()) > lim)
+                            return false;
+                }
+        }
+    return true;
+}
+
+// An axis on which source and target coincide but whose transform is longer
+// than S + T (embedded) keeps its full branches in the layout handed in and
+// out, and mirror storage on the device: the longer circulant has the same
+// symmetry, so pass 3 reads half the G^ per such axis (self 100x60x44 on
+// (128,64,48), ComplexF32: 151 -> 21 MB of G^, pass 3 37 -> 20 us, the call
+// 110 -> 92 us).  Data read from a file is checked rather than trusted.
+AxisStore axis_store(const gla_opr_s& h, const std::vector<std::complex<double>>& fur, int a, bool made)
+{
+    const gla_dims& d = h.dims;
+    if (d.sym[a]) return AxisStore{(int)d.fur_ext[a], d.fur_ext[a] != d.brn[a]};
+    const bool same = d.trg_cel[a] == d.src_cel[a] &&
+                      h.trg.org_num[a] * h.src.org_den[a] == h.src.org_num[a] * h.trg.org_den[a];
+    const int B = (int)d.dev_brn[a];
+    const bool half = same && d.dev_brn[a] != d.brn[a] && n_src_part(d) * n_trg_part(d) == 1 && B > 2 &&
+                      (made || mirrored(d, fur, a, d.dtype == GLA_C64 ? 1e-6 : 1e-12));
+    return half ? AxisStore{B / 2 + 1, true} : AxisStore{(int)d.fur_ext[a], false};
+}
+
 template <typename R>
-gla_status upload(gla_opr_t h, const std::vector<std::complex<double>>& furd)
+gla_status upload(gla_opr_t h, const std::vector<std::complex<double>>& furd, bool made)
 {
     using C = std::complex<R>;
     const gla_dims& d = h->dims;
-    const int64_t U0 = d.fur_ext[0], U1 = d.fur_ext[1], U2 = d.fur_ext[2];
-    const int64_t Ut = U0 * U1 * U2;
+    const int64_t F0 = d.fur_ext[0], F1 = d.fur_ext[1], Ft = F0 * F1 * d.fur_ext[2];
+    AxisStore as[3];
+    for (int a = 0; a < 3; ++a) as[a] = axis_store(*h, furd, a, made);
+    const int64_t U0 = as[0].U, U1 = as[1].U, U2 = as[2].U, Ut = U0 * U1 * U2;
     const int64_t P = n_src_part(d) * n_trg_part(d);
     const double scale = 1.0 / (double)(8 * d.dev_brn[0] * d.dev_brn[1] * d.dev_brn[2]);
     // device layout, one block per partition pair p = s + Ps * t:
-    // (((((p*8 + b)*U2 + j2)*U1 + j1)*U0 + j0)*6 + comp; the reference layout
-    // is ((b*P + p)*6 + comp)*Ut + j
+    // (((((p*8 + b)*U2 + j2)*U1 + j1)*U0 + j0)*6 + comp; the layout handed in
+    // is ((b*P + p)*6 + comp)*Ft + j
     std::vector<C> g((size_t)(P * 8 * Ut * 6));
     for (int64_t p = 0; p < P; ++p)
         for (int b = 0; b < 8; ++b)
             for (int c = 0; c < 6; ++c)
-                for (int64_t j = 0; j < Ut; ++j) {
-                    const std::complex<double> v = furd[(size_t)(((b * P + p) * 6 + c) * Ut + j)] * scale;
-                    g[(size_t)(((p * 8 + b) * Ut + j) * 6 + c)] = C((R)v.real(), (R)v.imag());
-                }
+                for (int64_t j2 = 0; j2 < U2; ++j2)
+                    for (int64_t j1 = 0; j1 < U1; ++j1) {
+                        const std::complex<double>* const in =
+                            &furd[(size_t)(((b * P + p) * 6 + c) * Ft + (j2 * F1 + j1) * F0)];
+                        C* const out = &g[(size_t)((((p * 8 + b) * U2 + j2) * U1 + j1) * U0 * 6 + c)];
+                        for (int64_t j0 = 0; j0 < U0; ++j0) {
+                            const std::complex<double> v = in[j0] * scale;
+                            out[6 * j0] = C((R)v.real(), (R)v.imag());
+                        }
+                    }
     // phase and twiddle tables per axis
     int64_t ntab = 0;
     for (int a = 0; a < 3; ++a) ntab += 2 * d.dev_brn[a];
@@ -378,9 +440,9 @@ gla_status upload(gla_opr_t h, const std::vector<std::complex<double>>& furd)
     for (int a = 0; a < 3; ++a) {
         gla::AxisMap& m = h->tab.am[a];
         m.B = (int)d.dev_brn[a];
-        m.U = (int)d.fur_ext[a];
-        m.sym = (d.sym[a] && d.fur_ext[a] != d.brn[a]) ? 1 : 0;
-        const int T = (int)d.trg_cel[a];
+        m.U = as[a].U;
+        m.sym = as[a].sym ? 1 : 0;
+        const int T = d.sym[a] ? (int)d.trg_cel[a] : m.B;
         m.fe = (T + 1) / 2 + (T % 2 == 0 ? 1 : 0);
         m.fo = (T + 1) / 2;
     }
@@ -595,7 +657,7 @@ bool finite_all(const T* p, int64_t n)
 
 namespace {
 gla_status create_common(const gla_opts* opts, const gla_vol* trg, const gla_vol* src, gla_dims d, const void* fur,
-                         int32_t fur_dtype, int64_t fur_len, gla_opr_t* out);
+                         int32_t fur_dtype, int64_t fur_len, bool made, gla_opr_t* out);
 }
 
 extern "C" {
@@ -618,7 +680,7 @@ gla_status gla_opr_create_from_fur(const gla_opts* opts, const gla_vol* trg, con
     if ((s = dims_impl(&t2, sp, DIMS_EXACT, &d))) return s;
     bool same = true;
     for (int a = 0; a < 3; ++a) same = same && d.dev_brn[a] == ref.brn[a];
-    if (same) return create_common(opts, &t2, sp, d, fur, fur_dtype, fur_len, out);
+    if (same) return create_common(opts, &t2, sp, d, fur, fur_dtype, fur_len, true, out);
     // a branch length without a compiled transform: the data is re-expressed
     // at the next fast length (gla::refur) in FP64
     const int64_t Ut = ref.fur_ext[0] * ref.fur_ext[1] * ref.fur_ext[2];
@@ -638,15 +700,17 @@ gla_status gla_opr_create_from_fur(const gla_opts* opts, const gla_vol* trg, con
         DevGuard g(opts->device);
         if ((s = gla::refur(ref, d, furd, re, err))) return fail(s, err);
     }
-    return create_common(opts, &t2, sp, d, re.data(), GLA_C128, (int64_t)re.size(), out);
+    return create_common(opts, &t2, sp, d, re.data(), GLA_C128, (int64_t)re.size(), true, out);
 }
 
 }  // extern "C"
 
 namespace {
 
+// made: the branches come from this library's own setup or re-embedding, so
+// an embedded axis's mirror symmetry needs no check
 gla_status create_common(const gla_opts* opts, const gla_vol* trg, const gla_vol* src, gla_dims d, const void* fur,
-                         int32_t fur_dtype, int64_t fur_len, gla_opr_t* out)
+                         int32_t fur_dtype, int64_t fur_len, bool made, gla_opr_t* out)
 {
     gla_status s;
     const int64_t Ut = d.fur_ext[0] * d.fur_ext[1] * d.fur_ext[2];
@@ -677,7 +741,7 @@ gla_status create_common(const gla_opts* opts, const gla_vol* trg, const gla_vol
     fill_geom(h.get());
     {
         DevGuard g(opts->device);
-        s = opts->dtype == GLA_C64 ? upload<float>(h.get(), furd) : upload<double>(h.get(), furd);
+        s = opts->dtype == GLA_C64 ? upload<float>(h.get(), furd, made) : upload<double>(h.get(), furd, made);
         if (s) return s;
     }
     // host copy in the operator's element type, rounded as the reference's
@@ -718,7 +782,7 @@ gla_status gla_opr_create(const gla_opts* opts, const gla_vol* trg, const gla_vo
     std::string err;
     s = gla::setup_fur(*opts, t2, sp ? s2 : t2, d, fur, err);
     if (s) return fail(s, err);
-    return create_common(opts, &t2, sp, d, fur.data(), GLA_C128, (int64_t)fur.size(), out);
+    return create_common(opts, &t2, sp, d, fur.data(), GLA_C128, (int64_t)fur.size(), true, out);
 }
 
 gla_status gla_opr_export_fur(gla_opr_t h, void* buf, int64_t len)
@@ -890,7 +954,7 @@ gla_status gla_opr_load(const char* path, int32_t dtype, int32_t device, gla_opr
     if (o.dtype != GLA_C64 && o.dtype != GLA_C128) return fail(GLA_ERR_TYPE, "dtype must be 0, GLA_C64 or GLA_C128");
     gla_status s = gla_init(device);
     if (s) return s;
-    return create_common(&o, &hd.trg, sp, d, pay.data(), hd.dtype, (int64_t)want, out);
+    return create_common(&o, &hd.trg, sp, d, pay.data(), hd.dtype, (int64_t)want, false, out);
 }
 
 gla_status gla_opr_adjoint(gla_opr_t h, gla_opr_t* out)
@@ -1100,7 +1164,7 @@ void pass_bytes(gla_opr_t h, int64_t nrhs, int64_t* bytes)
     const int64_t S = (int64_t)G.S[0] * G.S[1] * G.S[2], T = (int64_t)G.T[0] * G.T[1] * G.T[2];
     const int64_t a1 = (int64_t)G.L[0] * G.S[1] * G.S[2], a2 = (int64_t)G.L[0] * G.L[1] * G.S[2];
     const int64_t a3 = (int64_t)G.L[0] * G.L[1] * G.T[2], a4 = (int64_t)G.L[0] * G.T[1] * G.T[2];
-    const int64_t gsz = 8 * h->dims.fur_ext[0] * h->dims.fur_ext[1] * h->dims.fur_ext[2] * 6;
+    const int64_t gsz = 8LL * h->tab.am[0].U * h->tab.am[1].U * h->tab.am[2].U * 6;
     const int64_t f = 3 * nrhs * eb;
     bytes[0] = f * (S + a1);
     bytes[1] = f * (a1 + a2);
