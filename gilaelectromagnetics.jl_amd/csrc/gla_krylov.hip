@@ -24,7 +24,7 @@ namespace {
 
 constexpr int KT = 256;          // threads per chunk workgroup
 constexpr int KW = KT / 64;      // waves per chunk workgroup
-constexpr int KG = 8;            // basis vectors per sweep over a chunk
+constexpr int KG = 16;           // basis vectors per sweep over a chunk (2 KG sums, half a wave's lanes)
 
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -33,58 +33,73 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// elements per thread and sweep: every load of a sweep (the right-hand side
-// and up to KG basis vectors at E elements) is issued before the first use,
-// so a wave keeps (KG + 1) E loads in flight instead of one
-template <typename R> struct KE { static constexpr int value = 2; };
-template <> struct KE<double> { static constexpr int value = 1; };
+// VW consecutive elements as one load (16 bytes where the addresses allow it,
+// see wide_ok)
+template <typename R, int VW>
+struct alignas(sizeof(cpx<R>) * VW) vec {
+    cpx<R> e[VW];
+};
 
 // one sweep over a chunk for G basis vectors i0 .. i0 + G - 1 (G = 0: the
-// norm of w alone).  A thread visits q = lo + t, lo + t + KT, ... in
-// ascending order whatever E is; out-of-chunk elements load from a valid
-// address and contribute zero.
-template <typename R, int G>
+// norm of w alone).  Every load of a step (w and the G vectors) is issued
+// before the first use; a thread visits units of VW elements q = lo + VW t,
+// lo + VW (t + KT), ... in ascending order.  A last partial unit (n odd,
+// VW == 2) goes element by element.
+template <typename R, int G, int VW>
 __device__ __forceinline__ void dots_sweep(const cpx<R>* __restrict__ vp, int64_t vv, int i0,
                                            const cpx<R>* __restrict__ wp, int64_t lo, int64_t hi, bool first,
                                            double (&acc)[2 * KG + 1])
 {
-    constexpr int E = KE<R>::value;
-    const cpx<R>* vg[G > 0 ? G : 1];
+    auto add = [&](const cpx<R>& b, const cpx<R>* a) {
+        if (first) acc[2 * KG] += (double)b.x * b.x + (double)b.y * b.y;
 #pragma unroll
-    for (int g = 0; g < G; ++g) vg[g] = vp + (int64_t)(i0 + g) * vv;
-    for (int64_t q0 = lo + threadIdx.x; q0 < hi; q0 += (int64_t)KT * E) {
-        int64_t qe[E];
-        bool ok[E];
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            ok[e] = q0 + (int64_t)e * KT < hi;
-            qe[e] = ok[e] ? q0 + (int64_t)e * KT : q0;
+        for (int g = 0; g < G; ++g) {
+            acc[2 * g] += (double)a[g].x * b.x + (double)a[g].y * b.y;      // conj(a) b
+            acc[2 * g + 1] += (double)a[g].x * b.y - (double)a[g].y * b.x;
         }
-        cpx<R> b[E];
-        cpx<R> a[G > 0 ? G : 1][E];
+    };
+    const cpx<R>* const v0 = vp + (int64_t)i0 * vv;
+    int64_t q = lo + (int64_t)VW * threadIdx.x;
+    for (; q + VW <= hi; q += (int64_t)KT * VW) {
+        using V = vec<R, VW>;
+        const V b = *reinterpret_cast<const V*>(wp + q);
+        V a[G > 0 ? G : 1];
 #pragma unroll
-        for (int e = 0; e < E; ++e) b[e] = wp[qe[e]];
+        for (int g = 0; g < G; ++g) a[g] = *reinterpret_cast<const V*>(v0 + g * vv + q);
+        __builtin_amdgcn_sched_barrier(0);   // keep the step's loads ahead of the arithmetic
 #pragma unroll
-        for (int g = 0; g < G; ++g)
+        for (int e = 0; e < VW; ++e) {
+            cpx<R> ae[G > 0 ? G : 1];
 #pragma unroll
-            for (int e = 0; e < E; ++e) a[g][e] = vg[g][qe[e]];
-        __builtin_amdgcn_sched_barrier(0);   // keep the sweep's loads ahead of the arithmetic
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            if (!ok[e]) b[e] = cpx<R>{R(0), R(0)};
-            if (first) acc[2 * KG] += (double)b[e].x * b[e].x + (double)b[e].y * b[e].y;
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                acc[2 * g] += (double)a[g][e].x * b[e].x + (double)a[g][e].y * b[e].y;      // conj(a) b
-                acc[2 * g + 1] += (double)a[g][e].x * b[e].y - (double)a[g][e].y * b[e].x;
-            }
+            for (int g = 0; g < G; ++g) ae[g] = a[g].e[e];
+            add(b.e[e], ae);
         }
+    }
+    if (VW > 1 && q < hi) {
+        cpx<R> ae[G > 0 ? G : 1];
+#pragma unroll
+        for (int g = 0; g < G; ++g) ae[g] = v0[g * vv + q];
+        add(wp[q], ae);
     }
 }
 
-// part layout: [r][slot][chunk]; slots 0..nv-1 the dots, slot nv the squared
-// norm of w (when requested)
-template <typename R>
+template <typename R, int VW, int G>
+__device__ __forceinline__ void dots_count(int count, const cpx<R>* __restrict__ vp, int64_t vv, int i0,
+                                           const cpx<R>* __restrict__ wp, int64_t lo, int64_t hi, bool first,
+                                           double (&acc)[2 * KG + 1])
+{
+    if (count == G) dots_sweep<R, G, VW>(vp, vv, i0, wp, lo, hi, first, acc);
+    else if constexpr (G > 0) dots_count<R, VW, G - 1>(count, vp, vv, i0, wp, lo, hi, first, acc);
+}
+
+// Block products of one chunk.  part layout: [r][slot][chunk]; slots 0..nv-1
+// the dots, slot nv the squared norm of w (when requested).  Bound by HBM:
+// each right-hand side's basis is read once (8 right-hand sides, 16 vectors
+// of 3 x 64 x 64 x 48 ComplexF32 elements, 640 MB: 111 us with its sums, 5.8
+// TB/s where a bare read of the basis takes 97).  Before, with 8 vectors a
+// sweep, 8-byte loads, one wave sum per value and 4096-element chunks, it
+// took 129 us, and 8 x 98304 elements 34 us (now 21).
+template <typename R, int VW>
 __global__ __launch_bounds__(KT) void k_dots(const cpx<R>* __restrict__ V, int64_t vr, int64_t vv,
                                              const cpx<R>* __restrict__ w, int64_t wr, int64_t n, int nv,
                                              const int64_t* __restrict__ ncol, int64_t chunk, int nchunk, int nslot,
@@ -106,33 +121,35 @@ __global__ __launch_bounds__(KT) void k_dots(const cpx<R>* __restrict__ V, int64
 #pragma unroll
         for (int g = 0; g < 2 * KG + 1; ++g) acc[g] = 0.0;
         const bool first = i0 == 0 && self;
-        switch (nvr - i0 < KG ? nvr - i0 : KG) {
-        case 8: dots_sweep<R, 8>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        case 7: dots_sweep<R, 7>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        case 6: dots_sweep<R, 6>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        case 5: dots_sweep<R, 5>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        case 4: dots_sweep<R, 4>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        case 3: dots_sweep<R, 3>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        case 2: dots_sweep<R, 2>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        case 1: dots_sweep<R, 1>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        default: dots_sweep<R, 0>(vp, vv, i0, wp, lo, hi, first, acc); break;
-        }
+        const int count = nvr - i0 < KG ? nvr - i0 : KG;
+        dots_count<R, VW, KG>(count, vp, vv, i0, wp, lo, hi, first, acc);
+        // the wave's 2 KG sums, halving the values a lane carries at each step:
+        // lane l ends with value l / 2 (37 exchanges where a sum per value
+        // takes 192)
 #pragma unroll
-        for (int g = 0; g < 2 * KG + 1; ++g) {
-            const double v = wave_sum(acc[g]);
-            if (lane == 0) red[g][wv] = v;
+        for (int o = 32, hv = KG; o > 1; o >>= 1, hv >>= 1) {
+            const bool up = (lane & o) != 0;
+#pragma unroll
+            for (int g = 0; g < hv; ++g) {
+                const double keep = up ? acc[g + hv] : acc[g], give = up ? acc[g] : acc[g + hv];
+                acc[g] = keep + __shfl_xor(give, o);
+            }
+        }
+        acc[0] += __shfl_xor(acc[0], 1);
+        if ((lane & 1) == 0) red[lane >> 1][wv] = acc[0];
+        if (first) {
+            const double v = wave_sum(acc[2 * KG]);
+            if (lane == 0) red[2 * KG][wv] = v;
         }
         __syncthreads();
         if (threadIdx.x < 2 * KG + 1) {
             const int g = threadIdx.x;
-            double sum = 0.0;
+            if (g < 2 * KG ? g < 2 * count : first) {
+                double sum = 0.0;
 #pragma unroll
-            for (int u = 0; u < KW; ++u) sum += red[g][u];
-            if (g < 2 * KG) {
-                const int i = i0 + g / 2;
-                if (i < nvr) pr[((int64_t)i * 2 + (g & 1)) * nchunk + c] = sum;
-            } else if (first) {
-                pr[((int64_t)nv * 2) * nchunk + c] = sum;
+                for (int u = 0; u < KW; ++u) sum += red[g][u];
+                const int64_t slot = g < 2 * KG ? ((int64_t)i0 * 2 + g) : (int64_t)nv * 2;
+                pr[slot * nchunk + c] = sum;
             }
         }
         __syncthreads();
@@ -145,17 +162,21 @@ constexpr int KU = 4;
 // w[r] += s sum_i h[r][i] V[r][i] over one chunk; the chunk's squared norm
 // of the result goes to part[r][0][chunk] when norm is set.  Each element
 // sums its nv terms in order i = 0, 1, ...; a thread visits its elements in
-// ascending order (E at a time).
-template <typename R>
+// ascending order (E units of VW elements at a time).  Right-hand sides run
+// last to first: the products before it read the basis first to last, so the
+// end of it is still in the last-level cache (products and update of the
+// same case together: 264 us first to last, 231 last to first).
+template <typename R, int VW>
 __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64_t vr, int64_t vv,
                                              const cpx<double>* __restrict__ h, int64_t hr,
                                              cpx<R>* __restrict__ w, int64_t wr, int64_t n, int nv,
                                              const int64_t* __restrict__ ncol, double s, int64_t chunk, int nchunk,
                                              int norm, double* __restrict__ part)
 {
-    constexpr int E = KE<R>::value * 2;
+    constexpr int E = 2;
+    using U = vec<R, VW>;
     __shared__ double red[KW];
-    const int r = blockIdx.y, c = blockIdx.x;
+    const int r = gridDim.y - 1 - blockIdx.y, c = gridDim.x - 1 - blockIdx.x;
     if (ncol) nv = (int)(ncol[r] < 0 ? 0 : ncol[r] < nv ? ncol[r] : nv);
     const int64_t lo = (int64_t)c * chunk;
     const int64_t hi = lo + chunk < n ? lo + chunk : n;
@@ -163,56 +184,75 @@ __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64
     const cpx<double>* hp = h + r * hr;
     cpx<R>* wp = w + r * wr;
     double nrm = 0.0;
-    for (int64_t q0 = lo + threadIdx.x; q0 < hi; q0 += (int64_t)KT * E) {
+    auto finish = [&](cpx<R> o, double ar, double ai) {
+        const cpx<R> res{R((double)o.x + s * ar), R((double)o.y + s * ai)};
+        nrm += (double)res.x * res.x + (double)res.y * res.y;
+        return res;
+    };
+    const int64_t whole = lo + (hi - lo) / VW * VW;   // end of the whole units
+    for (int64_t q0 = lo + (int64_t)VW * threadIdx.x; q0 < whole; q0 += (int64_t)KT * E * VW) {
         int64_t qe[E];
         bool ok[E];
-        double ar[E], ai[E];
+        double ar[E][VW], ai[E][VW];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            ok[e] = q0 + (int64_t)e * KT < hi;
-            qe[e] = ok[e] ? q0 + (int64_t)e * KT : q0;
-            ar[e] = 0.0;
-            ai[e] = 0.0;
-        }
-        cpx<R> o[E];
+            ok[e] = q0 + (int64_t)e * KT * VW < whole;
+            qe[e] = ok[e] ? q0 + (int64_t)e * KT * VW : q0;
 #pragma unroll
-        for (int e = 0; e < E; ++e) o[e] = wp[qe[e]];
+            for (int k = 0; k < VW; ++k) ar[e][k] = ai[e][k] = 0.0;
+        }
+        U o[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) o[e] = *reinterpret_cast<const U*>(wp + qe[e]);
+        auto mac = [&](const cpx<double>& cc, int e, const U& a) {
+#pragma unroll
+            for (int k = 0; k < VW; ++k) {
+                ar[e][k] += cc.x * a.e[k].x - cc.y * a.e[k].y;
+                ai[e][k] += cc.x * a.e[k].y + cc.y * a.e[k].x;
+            }
+        };
         int i = 0;
         for (; i + KU <= nv; i += KU) {
-            cpx<R> a[KU][E];
+            U a[KU][E];
 #pragma unroll
             for (int u = 0; u < KU; ++u)
 #pragma unroll
-                for (int e = 0; e < E; ++e) a[u][e] = vp[(int64_t)(i + u) * vv + qe[e]];
+                for (int e = 0; e < E; ++e)
+                    a[u][e] = *reinterpret_cast<const U*>(vp + (int64_t)(i + u) * vv + qe[e]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int u = 0; u < KU; ++u) {
                 const cpx<double> cc = hp[i + u];
 #pragma unroll
-                for (int e = 0; e < E; ++e) {
-                    ar[e] += cc.x * a[u][e].x - cc.y * a[u][e].y;
-                    ai[e] += cc.x * a[u][e].y + cc.y * a[u][e].x;
-                }
+                for (int e = 0; e < E; ++e) mac(cc, e, a[u][e]);
             }
         }
         for (; i < nv; ++i) {
-            cpx<R> a[E];
+            U a[E];
 #pragma unroll
-            for (int e = 0; e < E; ++e) a[e] = vp[(int64_t)i * vv + qe[e]];
+            for (int e = 0; e < E; ++e) a[e] = *reinterpret_cast<const U*>(vp + (int64_t)i * vv + qe[e]);
             const cpx<double> cc = hp[i];
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                ar[e] += cc.x * a[e].x - cc.y * a[e].y;
-                ai[e] += cc.x * a[e].y + cc.y * a[e].x;
-            }
+            for (int e = 0; e < E; ++e) mac(cc, e, a[e]);
         }
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             if (!ok[e]) continue;
-            const cpx<R> res{R((double)o[e].x + s * ar[e]), R((double)o[e].y + s * ai[e])};
-            wp[qe[e]] = res;
-            nrm += (double)res.x * res.x + (double)res.y * res.y;
+            U res;
+#pragma unroll
+            for (int k = 0; k < VW; ++k) res.e[k] = finish(o[e].e[k], ar[e][k], ai[e][k]);
+            *reinterpret_cast<U*>(wp + qe[e]) = res;
         }
+    }
+    if (VW > 1 && whole < hi && threadIdx.x == 0) {
+        double ar = 0.0, ai = 0.0;
+        for (int i = 0; i < nv; ++i) {
+            const cpx<R> a = vp[(int64_t)i * vv + whole];
+            const cpx<double> cc = hp[i];
+            ar += cc.x * a.x - cc.y * a.y;
+            ai += cc.x * a.y + cc.y * a.x;
+        }
+        wp[whole] = finish(wp[whole], ar, ai);
     }
     if (!norm) return;   // uniform over the launch
     nrm = wave_sum(nrm);
@@ -225,6 +265,23 @@ __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64
         for (int u = 0; u < KW; ++u) sum += red[u];
         part[(int64_t)r * nchunk + c] = sum;
     }
+}
+
+// The chunk sums of the products, one wave per output as k_chunk_sum, written
+// where they belong: slot i < nv of right-hand side r to h[r nv + i] (re, im
+// by row parity), slot nv to w2[r].
+__global__ __launch_bounds__(64) void k_dots_sum(const double* __restrict__ part, int nchunk, int nv,
+                                                 double* __restrict__ h, double* __restrict__ w2)
+{
+    const int row = blockIdx.x, r = blockIdx.y;
+    if (row >= 2 * nv && (row > 2 * nv || !w2)) return;
+    const double* const p = part + ((int64_t)r * (nv + 1) * 2 + row) * nchunk;
+    double v = 0.0;
+    for (int c = threadIdx.x; c < nchunk; c += 64) v += p[c];
+    v = wave_sum(v);
+    if (threadIdx.x != 0) return;
+    if (row < 2 * nv) h[(int64_t)r * 2 * nv + row] = v;
+    else w2[r] = v;
 }
 
 // out[j] = sum over chunks of part[j][chunk], one wave per output: lane l sums
@@ -284,10 +341,21 @@ __global__ __launch_bounds__(256) void k_next(cpx<R>* __restrict__ V, int64_t vr
 int64_t krylov_chunk(int64_t n)
 {
     // about 1024 workgroups per right-hand side for long vectors, at least
-    // 4096 elements per workgroup
+    // 2048 elements per workgroup; even, so that a chunk starts on a whole
+    // 16-byte unit
     int64_t c = (n + 1023) / 1024;
-    if (c < 4096) c = 4096;
-    return c;
+    if (c < 2048) c = 2048;
+    return c + (c & 1);
+}
+
+// Whether rows at these element strides allow 16-byte loads: ComplexF32
+// pairs need even strides and aligned bases, ComplexF64 elements are 16
+// bytes themselves.
+template <typename R>
+static bool wide_ok(const void* V, int64_t vr, int64_t vv, const void* w, int64_t wr)
+{
+    if (sizeof(cpx<R>) == 16) return false;   // one element is a whole unit
+    return vr % 2 == 0 && vv % 2 == 0 && wr % 2 == 0 && (uintptr_t)V % 16 == 0 && (uintptr_t)w % 16 == 0;
 }
 
 int64_t krylov_part_doubles(int64_t k, int64_t nv, int64_t n)
@@ -306,27 +374,14 @@ hipError_t run_krylov_dots(int64_t k, int nv, int64_t n, const void* V, int64_t 
     const int nchunk = (int)((n + chunk - 1) / chunk);
     const int self = w2 != nullptr;
     const int nslot = nv + 1;
-    hipLaunchKernelGGL(k_dots<R>, dim3(nchunk, (unsigned)k), dim3(KT), 0, st, (const cpx<R>*)V, vr, vv,
+    const auto kernel = wide_ok<R>(V, vr, vv, w, wr) ? k_dots<R, sizeof(cpx<R>) == 8 ? 2 : 1> : k_dots<R, 1>;
+    hipLaunchKernelGGL(kernel, dim3(nchunk, (unsigned)k), dim3(KT), 0, st, (const cpx<R>*)V, vr, vv,
                        (const cpx<R>*)w, wr, n, nv, ncol, chunk, nchunk, nslot, self, (double*)part);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    // every (r, slot, re/im) row of part sums into h (re/im interleaved,
-    // h[r][i]) -- the slot-nv rows (norms) into a scratch tail of part
-    const int64_t rows = k * nslot * 2;
-    double* sums = (double*)part + rows * nchunk;
-    hipLaunchKernelGGL(k_chunk_sum, dim3((unsigned)rows), dim3(64), 0, st, (const double*)part, nchunk, rows, sums);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    // unpack: sums[(r*nslot + i)*2 + {0,1}] -> h[r*nv + i], norms -> w2[r]
-    if (nv > 0) {
-        e = hipMemcpy2DAsync(h, (size_t)nv * 16, sums, (size_t)nslot * 16, (size_t)nv * 16, (size_t)k,
-                             hipMemcpyDeviceToDevice, st);
-        if (e != hipSuccess) return e;
-    }
-    if (self)
-        e = hipMemcpy2DAsync(w2, sizeof(double), sums + (int64_t)nv * 2, (size_t)nslot * 16, sizeof(double),
-                             (size_t)k, hipMemcpyDeviceToDevice, st);
-    return e;
+    hipLaunchKernelGGL(k_dots_sum, dim3((unsigned)(2 * nv + self), (unsigned)k), dim3(64), 0, st, (const double*)part,
+                       nchunk, nv, (double*)h, w2);
+    return hipGetLastError();
 }
 
 template <typename R>
@@ -337,7 +392,10 @@ hipError_t run_krylov_axpy(int64_t k, int nv, int64_t n, const void* V, int64_t 
     const int64_t chunk = krylov_chunk(n);
     const int nchunk = (int)((n + chunk - 1) / chunk);
     const int norm = w2 != nullptr;
-    hipLaunchKernelGGL(k_axpy<R>, dim3(nchunk, (unsigned)k), dim3(KT), 0, st, (const cpx<R>*)V, vr, vv,
+    const auto kernel = wide_ok<R>(nv > 0 ? V : w, nv > 0 ? vr : 0, nv > 0 ? vv : 0, w, wr)
+                            ? k_axpy<R, sizeof(cpx<R>) == 8 ? 2 : 1>
+                            : k_axpy<R, 1>;
+    hipLaunchKernelGGL(kernel, dim3(nchunk, (unsigned)k), dim3(KT), 0, st, (const cpx<R>*)V, vr, vv,
                        (const cpx<double>*)h, hr, (cpx<R>*)w, wr, n, nv, ncol, s, chunk, nchunk, norm,
                        (double*)part);
     hipError_t e = hipGetLastError();
