@@ -16,6 +16,7 @@
 
 #include "gla_krylov.hpp"
 #include "gla_launch.hpp"
+#include "gla_planes.hpp"
 #include "gla_setup.hpp"
 
 namespace {
@@ -1086,6 +1087,8 @@ gla_status gla_opr_apply_host(gla_opr_t h, const void* x, int64_t nx, void* y, i
 namespace {
 gla_status profile_locked(gla_opr_t h, const void* x, void* y, int64_t nrhs, void* stream, int32_t reps, double* ms,
                           int64_t* bytes);
+gla_status profile_seq_locked(gla_opr_t h, const void* x, void* y, int64_t nrhs, void* stream, int32_t reps, double* ms,
+                              int64_t* bytes, double* total_ms);
 void pass_bytes(gla_opr_t h, int64_t nrhs, int64_t* bytes);
 }
 extern "C" {
@@ -1112,11 +1115,24 @@ gla_status gla_opr_profile_seq(gla_opr_t h, const void* x, int64_t nx, void* y, 
         return fail(GLA_ERR_UNSUPPORTED, "per-pass profiles cover operators with one partition pair");
     gla_status s = run(h, x, nx, y, ny, nrhs, 1, 0, 0, 0, 0, stream);   // validates, allocates, warms up
     if (s) return s;
+    s = profile_seq_locked(h, x, y, nrhs, stream, reps, ms, bytes, total_ms);
+    if (s) return s;
+    // leave y holding a plain apply's matvec (the plane kernels round differently)
+    return run(h, x, nx, y, ny, nrhs, 1, 0, 0, 0, 0, stream);
+}
+
+}  // extern "C"
+
+namespace {
+
+gla_status profile_seq_locked(gla_opr_t h, const void* x, void* y, int64_t nrhs, void* stream, int32_t reps, double* ms,
+                              int64_t* bytes, double* total_ms)
+{
     std::lock_guard<std::mutex> lk(h->mu);
     DevGuard g(h->opts.device);
     pass_bytes(h, nrhs, bytes);   // algorithmic bytes per pass, as gla_opr_profile
-    // reps matvecs exactly as gla_opr_apply issues them, with an event at
-    // every pass boundary: pass p of matvec r lasts ev[r][p] -> ev[r][p+1]
+    // reps matvecs of five launches each, with an event at every pass
+    // boundary: pass p of matvec r lasts ev[r][p] -> ev[r][p+1]
     const int ne = gla::NPASS + 1;
     std::vector<hipEvent_t> ev((size_t)reps * ne, nullptr);
     hipError_t e = hipSuccess;
@@ -1151,10 +1167,6 @@ gla_status gla_opr_profile_seq(gla_opr_t h, const void* x, int64_t nx, void* y, 
     *total_ms = (double)tot / reps;
     return GLA_OK;
 }
-
-}  // extern "C"
-
-namespace {
 
 // algorithmic HBM bytes of each pass of one matvec over nrhs right-hand sides
 void pass_bytes(gla_opr_t h, int64_t nrhs, int64_t* bytes)
@@ -1503,6 +1515,19 @@ gla_status gla_krylov_next(int32_t dtype, int64_t k, int64_t n, void* V, int64_t
 }  // extern "C"
 
 namespace gla {
+
+bool use_planes(const Geom& g, int complex_bytes, int slots)
+{
+    bool x = false, y = false;
+#define GLA_LEN_XY(k) x = x || g.B[0] == k, y = y || g.B[1] == k;
+    GLA_FOR_EACH_PLANE(GLA_LEN_XY)
+#undef GLA_LEN_XY
+    // a target much longer than B on axis 2 can make the inverse's plane
+    // larger than a CU's LDS
+    constexpr size_t lim = 140 * 1024;
+    return x && y && slots <= 65535 && plane_bytes(g, complex_bytes, false) <= lim &&
+           plane_bytes(g, complex_bytes, true) <= lim;
+}
 
 bool len_supported(int n)
 {

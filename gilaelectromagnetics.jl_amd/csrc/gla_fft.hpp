@@ -645,4 +645,40 @@ struct PencilFft {
     }
 };
 
+// LDS exchanges of the radix plan for N with E elements per thread
+__host__ __device__ constexpr int plan_exchanges(int N, int E, int pol)
+{
+    const Plan p = make_plan(N, E, pol);
+    if (p.nst <= 1) return (p.nst == 1 && E % p.rad[0] == 0) ? 0 : 1;
+    const bool fr = E % p.rad[0] == 0, lr = E % p.rad[p.nst - 1] == 0;
+    return (p.nst - 1) + (fr ? 0 : 1) + (lr ? 0 : 1);
+}
+
+// elements per thread: close to `target`, with few LDS exchanges, threads
+// per pencil within `maxtp` and, when `wave` is set, dividing 64 (a pencil
+// inside one wave) -- unless that would leave more than 64 elements per
+// thread (lengths with a large odd factor, e.g. 81, 145), in which case the
+// pencil spans waves (workgroup barriers) with at most 32 elements per thread
+__host__ __device__ constexpr int pick_e_in(int N, int target, int maxtp, bool wave, int emax, int pol)
+{
+    int best = 0, bestscore = 1 << 30;
+    for (int e = 1; e <= N; ++e) {
+        if (N % e) continue;
+        const int tp = N / e;
+        if (tp > maxtp || e > emax) continue;
+        const int d = e > target ? 2 * (e - target) : target - e;
+        const int score = d + 4 * plan_exchanges(N, e, pol) + ((wave && 64 % tp != 0) ? 1000 : 0);
+        if (score < bestscore) { bestscore = score; best = e; }
+    }
+    return best;
+}
+
+__host__ __device__ constexpr int pick_e(int N, int target, int maxtp, bool wave, int pol)
+{
+    const int e = pick_e_in(N, target, maxtp, wave, N, pol);
+    if (e > 0 && e <= 64) return e;
+    const int f = pick_e_in(N, target, maxtp, false, 32, pol);
+    return f > 0 ? f : (e > 0 ? e : N);
+}
+
 }  // namespace gla

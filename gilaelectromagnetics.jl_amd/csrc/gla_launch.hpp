@@ -69,6 +69,31 @@ bool len_supported(int n);
 bool len_fast(int n);             // 2^a x {1, 3, 5}: the lengths operators from geometry embed into
 int len_next_supported(int n);   // smallest fast length >= n, or 0
 
+// parities of a column that the plane kernels (gla_planes.hpp) transform
+// together, from the exchange buffers' size
+constexpr int plane_k(int complex_bytes, int cols, int n2) { return 2 * cols * n2 * complex_bytes <= 65536 ? 2 : 1; }
+
+// LDS of the plane kernels: the plane between the two transforms -- forward
+// one axis-1 parity, inverse both -- or the exchange buffers of its columns,
+// and the tables
+inline size_t plane_bytes(const Geom& g, int complex_bytes, bool inverse)
+{
+    const int cols = g.B[0] * (inverse ? 2 : 1), n = plane_k(complex_bytes, cols, g.B[1]) * g.B[1];
+    const int cells = inverse ? g.T[1] : g.S[1];
+    return (size_t)((cells > n ? cells : n) * cols + 2 * (g.B[0] + g.B[1])) * complex_bytes;
+}
+
+// whether passes 1 + 2 and 4 + 5 run as plane kernels (gla_planes.hpp) over
+// `slots` right-hand sides (times partitions)
+bool use_planes(const Geom& g, int complex_bytes, int slots);
+
+template <typename R>
+hipError_t run_fwd_planes(const Geom& g, const DevTab& tb, const void* X, void* W2, int slots, hipStream_t st);
+
+template <typename R>
+hipError_t run_inv_planes(const Geom& g, const DevTab& tb, const void* W2, void* Y, int slots, double ar, double ai,
+                          double br, double bi, int axpby, const Epi& epi, hipStream_t st);
+
 constexpr int NPASS = 5;
 
 // one pass of the pipeline: 0 x-forward, 1 y-forward, 2 z fused, 3 y-inverse,

@@ -40,44 +40,6 @@
 
 namespace gla {
 
-// elements per thread: the divisor of N closest to `target` from below,
-// raised until the workgroup fits in `maxtp` threads per pencil
-// LDS exchanges of the radix plan for N with E elements per thread
-__host__ __device__ constexpr int plan_exchanges(int N, int E, int pol)
-{
-    const Plan p = make_plan(N, E, pol);
-    if (p.nst <= 1) return (p.nst == 1 && E % p.rad[0] == 0) ? 0 : 1;
-    const bool fr = E % p.rad[0] == 0, lr = E % p.rad[p.nst - 1] == 0;
-    return (p.nst - 1) + (fr ? 0 : 1) + (lr ? 0 : 1);
-}
-
-// elements per thread: close to `target`, with few LDS exchanges, threads
-// per pencil within `maxtp` and, when `wave` is set, dividing 64 (a pencil
-// inside one wave) -- unless that would leave more than 64 elements per
-// thread (lengths with a large odd factor, e.g. 81, 145), in which case the
-// pencil spans waves (workgroup barriers) with at most 32 elements per thread
-__host__ __device__ constexpr int pick_e_in(int N, int target, int maxtp, bool wave, int emax, int pol)
-{
-    int best = 0, bestscore = 1 << 30;
-    for (int e = 1; e <= N; ++e) {
-        if (N % e) continue;
-        const int tp = N / e;
-        if (tp > maxtp || e > emax) continue;
-        const int d = e > target ? 2 * (e - target) : target - e;
-        const int score = d + 4 * plan_exchanges(N, e, pol) + ((wave && 64 % tp != 0) ? 1000 : 0);
-        if (score < bestscore) { bestscore = score; best = e; }
-    }
-    return best;
-}
-
-__host__ __device__ constexpr int pick_e(int N, int target, int maxtp, bool wave, int pol)
-{
-    const int e = pick_e_in(N, target, maxtp, wave, N, pol);
-    if (e > 0 && e <= 64) return e;
-    const int f = pick_e_in(N, target, maxtp, false, 32, pol);
-    return f > 0 ? f : (e > 0 ? e : N);
-}
-
 template <typename R>
 struct Cfg {
     static constexpr bool DBL = sizeof(R) == 8;
@@ -279,11 +241,12 @@ template <typename R>
 hipError_t run_matvec(const Geom& g, const DevTab& tb, const void* X, void* Y, void* W1, void* W2, int nrhs,
                       double ar, double ai, double br, double bi, int axpby, const Epi& epi, hipStream_t st)
 {
-    for (int p = 0; p < NPASS; ++p) {
-        hipError_t e = run_pass<R>(p, g, tb, X, Y, W1, W2, nrhs, ar, ai, br, bi, axpby, epi, st);
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
+    const bool planes = use_planes(g, (int)sizeof(cpx<R>), nrhs);
+    hipError_t e = planes ? run_fwd_planes<R>(g, tb, X, W2, nrhs, st) : hipSuccess;
+    for (int p = planes ? 2 : 0; p < (planes ? 3 : NPASS) && e == hipSuccess; ++p)
+        e = run_pass<R>(p, g, tb, X, Y, W1, W2, nrhs, ar, ai, br, bi, axpby, epi, st);
+    if (planes && e == hipSuccess) e = run_inv_planes<R>(g, tb, W2, Y, nrhs, ar, ai, br, bi, axpby, epi, st);
+    return e;
 }
 
 // pass 3 of a partitioned operator on the shape of pass 3; the thread groups
@@ -340,12 +303,20 @@ hipError_t run_matvec_parts(const Geom& g0, const DevTab& tb, const void* X, voi
     void* Wo = W2;
     if (Pt == 1) go.w2s = (int64_t)Ps * g.w2s;
     else Wo = (cpx<R>*)W2 + (int64_t)nrhs * Ps * g.w2s;
-    hipError_t e = run_pass<R>(0, g, tb, X, Y, W1, W2, nrhs, ar, ai, br, bi, axpby, Epi(), st);
-    if (e == hipSuccess) e = run_pass<R>(1, g, tb, X, Y, W1, W2, nrhs * Ps, ar, ai, br, bi, axpby, Epi(), st);
+    constexpr int CB = (int)sizeof(cpx<R>);
+    hipError_t e;
+    if (use_planes(g, CB, nrhs * Ps)) {
+        e = run_fwd_planes<R>(g, tb, X, W2, nrhs * Ps, st);
+    } else {
+        e = run_pass<R>(0, g, tb, X, Y, W1, W2, nrhs, ar, ai, br, bi, axpby, Epi(), st);
+        if (e == hipSuccess) e = run_pass<R>(1, g, tb, X, Y, W1, W2, nrhs * Ps, ar, ai, br, bi, axpby, Epi(), st);
+    }
     if (e != hipSuccess) return e;
 #define GLA_CASE_3(n) case n: e = launch_zpart<R, n>(g, tb, W2, Wo, go.w2s, nrhs, Ps, Pt, gpair, st); break;
     switch (g.B[2]) { GLA_FOR_EACH_LEN(GLA_CASE_3) default: return hipErrorInvalidValue; }
 #undef GLA_CASE_3
+    if (e == hipSuccess && use_planes(go, CB, nrhs * Pt))
+        return run_inv_planes<R>(go, tb, Wo, Y, nrhs * Pt, ar, ai, br, bi, axpby, Epi(), st);
     if (e == hipSuccess) e = run_pass<R>(3, go, tb, X, Y, W1, Wo, nrhs * Pt, ar, ai, br, bi, axpby, Epi(), st);
     if (e == hipSuccess) e = run_pass<R>(4, g, tb, X, Y, W1, W2, nrhs, ar, ai, br, bi, axpby, Epi(), st);
     return e;

@@ -1,0 +1,5 @@
+// Plane kernels (passes 1 + 2 and 4 + 5 of small planes), R = double.
+#include "gla_planes_impl.hpp"
+template hipError_t gla::run_fwd_planes<double>(const gla::Geom&, const gla::DevTab&, const void*, void*, int, hipStream_t);
+template hipError_t gla::run_inv_planes<double>(const gla::Geom&, const gla::DevTab&, const void*, void*, int, double,
+                                            double, double, double, int, const gla::Epi&, hipStream_t);

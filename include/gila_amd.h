@@ -221,9 +221,10 @@ gla_status gla_opr_apply_host(gla_opr_t h, const void* x, int64_t nx, void* y, i
 gla_status gla_opr_profile(gla_opr_t h, const void* x, int64_t nx, void* y, int64_t ny, int64_t nrhs, void* stream,
                            int32_t reps, double* ms, int64_t* bytes);
 
-/* The same figures measured inside the real sequence: `reps` matvecs issued
- * exactly as gla_opr_apply issues them, with an event at every pass
- * boundary; ms[p] is pass p's average duration between its boundary events,
+/* The same figures measured inside the real sequence: `reps` matvecs of the
+ * five passes, issued as gla_opr_apply issues them (which runs passes 0 and 1,
+ * and 3 and 4, of planes up to 64 x 64 branch points as one kernel each; here
+ * they are timed apart), with an event at every pass boundary; ms[p] is pass p's average duration between its boundary events,
  * bytes[p] its algorithmic HBM bytes and *total_ms the average duration of
  * one whole matvec over the run.  Synchronizes; y holds a valid matvec on
  * return.  No counterpart in the reference; for benchmarks. */
