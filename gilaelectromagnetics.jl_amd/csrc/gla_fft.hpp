@@ -559,12 +559,18 @@ struct PencilFft {
         }
     }
 
+    // late() is called before the last stage: a point where a caller can issue
+    // loads that the stage hides and whose registers the earlier ones did not
+    // have to spare
+    template <typename Late>
     static __device__ __forceinline__ void run(cpx<R> (&v)[K][E], cpx<R>* lds, int t, int pen,
-                                               const cpx<R>* __restrict__ tw)
+                                               const cpx<R>* __restrict__ tw, Late late)
     {
         if constexpr (P.nst == 0) {
+            late();
             return;
         } else if constexpr (P.nst == 1 && FIRST_REG) {
+            late();
             // whole transform inside one thread (E == N)
 #pragma unroll
             for (int k = 0; k < K; ++k) dft<R, INV, P.rad[0], N>(v[k], tw);
@@ -595,6 +601,7 @@ struct PencilFft {
                 lds_sync<SYNC>();
                 mid_stages<0>(lds, t, pen, tw);
             }
+            late();
             // ---- last stage
             if constexpr (LAST_REG) {
                 constexpr int S = P.nst - 1;
@@ -634,6 +641,12 @@ struct PencilFft {
             }
             lds_sync<SYNC>();   // LDS free for the next transform
         }
+    }
+
+    static __device__ __forceinline__ void run(cpx<R> (&v)[K][E], cpx<R>* lds, int t, int pen,
+                                               const cpx<R>* __restrict__ tw)
+    {
+        run(v, lds, t, pen, tw, [] {});
     }
 
     // single pencil

@@ -618,6 +618,12 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_zpass(cpx<R>* __restrict__ W2
     // first point's loads issued before the forward transform (pre_g), so
     // they arrive during its stages
     constexpr bool GPIPE = (GG & 2) != 0, GPRE = GPIPE && (GG & 4) != 0;
+    // bit 3 (with KB == 3): every point's loads issued ahead -- the first
+    // GEARLY before the forward transform, the others before its last stage
+    constexpr bool GALL = (GG & 8) != 0 && KB == 3;
+    constexpr int GEARLY = GPRE ? 1 : 0;
+    cpx<R> ga[GALL ? E : 1][6];
+    R gas[GALL ? E : 1];
     cpx<R> g0[6];
     R g0s = R(1);
     auto gbase = [&](int p3) {
@@ -628,15 +634,36 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_zpass(cpx<R>* __restrict__ W2
     // stored entry), so the wait for the column data before the forward
     // transform can leave these loads in flight
     auto pre_g = [&](int p3) {
-        if constexpr (GPRE) g_fetch<R, TP>(gbase(p3), uu, a3, p3, t, 0, g0, g0s);
+        if constexpr (GALL && GEARLY > 0) g_fetch<R, TP>(gbase(p3), uu, a3, p3, t, 0, ga[0], gas[0]);
+        else if constexpr (GPRE) g_fetch<R, TP>(gbase(p3), uu, a3, p3, t, 0, g0, g0s);
     };
     auto mul_g = [&](cpx<R>(&w)[3][E], int p3) {
+        if constexpr (GALL) {
+            if (!act) return;
+            const R s12 = R(s1 * s2);
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const cpx<R>(&g)[6] = ga[e];
+                const R s13 = R(s1) * gas[e], s23 = R(s2) * gas[e];
+                const cpx<R> gxy = s12 * g[3], gxz = s13 * g[4], gyz = s23 * g[5];
+                const cpx<R> x0 = w[0][e], x1 = w[1][e], x2 = w[2][e];
+                w[0][e] = g[0] * x0 + gxy * x1 + gxz * x2;
+                w[1][e] = gxy * x0 + g[1] * x1 + gyz * x2;
+                w[2][e] = gxz * x0 + gyz * x1 + g[2] * x2;
+            }
+            return;
+        }
         g_multiply<R, E, TP, GPIPE>(w, gbase(p3), uu, a3, p3, t, s1, s2, act, GPRE ? &g0 : nullptr, g0s);
     };
     const cpx<R>* twu = (GG & 1) ? twl : tw;
     const cpx<R>* phu = (GG & 1) ? twl + N : phz;
-    auto fwd = [&](cpx<R>(&w)[3][E]) {
-        if constexpr (KB == 3) {
+    auto fwd = [&](cpx<R>(&w)[3][E], int p3) {
+        if constexpr (GALL) {
+            FftF3::run(w, lds, t, xl, twu, [&] {
+#pragma unroll
+                for (int e = GEARLY; e < E; ++e) g_fetch<R, TP>(gbase(p3), uu, a3, p3, t, e, ga[e], gas[e]);
+            });
+        } else if constexpr (KB == 3) {
             FftF3::run(w, lds, t, xl, twu);
         } else {
 #pragma unroll
@@ -672,11 +699,11 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_zpass(cpx<R>* __restrict__ W2
                 }
             }
         pre_g(0);
-        fwd(wv[0]);
+        fwd(wv[0], 0);
         mul_g(wv[0], 0);
         inv(wv[0]);
         pre_g(1);
-        fwd(wv[1]);
+        fwd(wv[1], 1);
         mul_g(wv[1], 1);
         inv(wv[1]);
         if (!act) return;
@@ -718,7 +745,7 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_zpass(cpx<R>* __restrict__ W2
                 else w[c][e] = p3 == 0 ? a : phu[n] * a;   // no spill-over half
             }
         pre_g(p3);
-        fwd(w);
+        fwd(w, p3);
         mul_g(w, p3);
         inv(w);
 #pragma unroll

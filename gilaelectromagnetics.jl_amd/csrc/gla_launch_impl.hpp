@@ -171,8 +171,8 @@ static hipError_t launch_zpass(const Geom& g, const DevTab& tb, void* W2, int nr
     const int maxr = (int)(lim < 1 ? 1 : (lim < nrhs ? lim : nrhs));
     for (int r0 = 0; r0 < nrhs; r0 += maxr) {
         const int cnt = nrhs - r0 < maxr ? nrhs - r0 : maxr;
-        const bool small = (int64_t)g.L[0] * g.L[1] < ZSMALL_COLS;
         cpx<R>* const w = (cpx<R>*)W2 + (int64_t)r0 * g.w2s;
+        const bool small = (int64_t)g.L[0] * g.L[1] < ZSMALL_COLS;
         const hipError_t e = small ? launch_zpass_shape<R, N, 1>(g, tb, w, cnt, st)
                                    : launch_zpass_shape<R, N, 0>(g, tb, w, cnt, st);
         if (e != hipSuccess) return e;

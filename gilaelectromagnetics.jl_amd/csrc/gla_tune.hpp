@@ -18,7 +18,12 @@
 //          parities split first
 //   gtune: pass 3's G^ loads -- 3: root and phase tables in LDS and the G^
 //          loads pipelined one point ahead; 7: also the first point's loads
-//          issued before the forward transform (more registers)
+//          issued before the forward transform (more registers); 15: and every
+//          other point's before its last stage (ComplexF64 lengths of four
+//          elements a thread, whose two waves per SIMD have the registers and
+//          wait on these loads otherwise: pass 3 at 128^3 311 -> 299 us, on
+//          128x80x80 branch points 157 -> 143, 64x64x160 147 -> 135; 96, two
+//          elements a thread, 140 -> 150, ComplexF32 128^3 153 -> 179)
 //   ptune: the radix plan of every pencil transform of that length -- 0 takes
 //          the largest radices (fewest LDS exchanges), 1 only radices that
 //          divide the elements per thread (every thread busy in every stage,
@@ -215,6 +220,10 @@ constexpr int gtune(int complex_bytes, int n)
 #else
     switch (n) {
         // BEGIN TUNED GG C128
+            case 64: return 15;
+            case 80: return 15;
+            case 128: return 15;
+            case 160: return 15;
             case 320: return 7;
         // END TUNED GG C128
         default: return 3;
@@ -275,6 +284,10 @@ constexpr int ltune(int complex_bytes, int n)
 #else
     switch (n) {
         // BEGIN TUNED RELOAD C128
+            case 64: return 0;
+            case 80: return 0;
+            case 128: return 0;
+            case 160: return 0;
         // END TUNED RELOAD C128
         default: return 2;
     }
