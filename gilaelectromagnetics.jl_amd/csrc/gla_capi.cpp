@@ -1539,7 +1539,7 @@ bool len_supported(int n)
 
 int zpass_tile_width(int complex_bytes, int n, int L1, int L2)
 {
-    return ztune(complex_bytes, n, (int64_t)L1 * L2 < ZSMALL_COLS).px;
+    return ztile(complex_bytes, n, (int64_t)L1 * L2 < ZSMALL_COLS);
 }
 
 std::vector<int> zpass_order(const int B[3], const int L[3], const AxisMap am[3], int px)

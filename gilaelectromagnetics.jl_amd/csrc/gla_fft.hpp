@@ -215,6 +215,35 @@ __device__ __forceinline__ void dft16(cpx<R>* a)
     }
 }
 
+// radix P Q with P, Q coprime (prime-factor map, no twiddles): input
+// n = (Q n1 + P n2) mod PQ, output k = (Q (Q^-1 mod P) k1 + P (P^-1 mod Q) k2) mod PQ
+template <typename R, bool INV, int RAD, int N>
+__device__ __forceinline__ void dft(cpx<R>* a, const cpx<R>* __restrict__ tw);
+
+template <typename R, bool INV, int P, int Q>
+__device__ __forceinline__ void dft_pq(cpx<R>* a)
+{
+    constexpr int M = P * Q;
+    constexpr int ip = [] { for (int i = 1; i < P; ++i) if ((Q * i) % P == 1) return i; return 1; }();   // Q^-1 mod P
+    constexpr int iq = [] { for (int i = 1; i < Q; ++i) if ((P * i) % Q == 1) return i; return 1; }();   // P^-1 mod Q
+    cpx<R> b[Q][P];
+#pragma unroll
+    for (int n2 = 0; n2 < Q; ++n2) {
+#pragma unroll
+        for (int n1 = 0; n1 < P; ++n1) b[n2][n1] = a[(Q * n1 + P * n2) % M];
+        dft<R, INV, P, P>(b[n2], nullptr);
+    }
+#pragma unroll
+    for (int k1 = 0; k1 < P; ++k1) {
+        cpx<R> c[Q];
+#pragma unroll
+        for (int n2 = 0; n2 < Q; ++n2) c[n2] = b[n2][k1];
+        dft<R, INV, Q, Q>(c, nullptr);
+#pragma unroll
+        for (int k2 = 0; k2 < Q; ++k2) a[(Q * ip * k1 + P * iq * k2) % M] = c[k2];
+    }
+}
+
 // generic odd radix: direct sum over the pairs (e, RAD - e), whose roots are
 // conjugate: with s_e = a_e + a_{RAD-e}, d_e = a_e - a_{RAD-e} and
 // w^{eq} = C + i S,
@@ -266,7 +295,10 @@ __device__ __forceinline__ void dft(cpx<R>* a, const cpx<R>* __restrict__ tw)
     else if constexpr (RAD == 3) dft3<R, INV>(a);
     else if constexpr (RAD == 4) dft4<R, INV>(a);
     else if constexpr (RAD == 5) dft5<R, INV>(a);
+    else if constexpr (RAD == 6) dft_pq<R, INV, 2, 3>(a);
     else if constexpr (RAD == 8) dft8<R, INV>(a);
+    else if constexpr (RAD == 10) dft_pq<R, INV, 2, 5>(a);
+    else if constexpr (RAD == 12) dft_pq<R, INV, 4, 3>(a);
     else if constexpr (RAD == 16) dft16<R, INV>(a);
     else dftg<R, INV, RAD, N>(a, tw);
 }
@@ -693,5 +725,166 @@ __host__ __device__ constexpr int pick_e(int N, int target, int maxtp, bool wave
     const int f = pick_e_in(N, target, maxtp, false, 32, pol);
     return f > 0 ? f : (e > 0 ? e : N);
 }
+
+// Makes a table pointer opaque to the compiler, so the values read through it
+// are read again at each use instead of being kept in registers from an
+// earlier one.
+template <typename T>
+__device__ __forceinline__ void reread(T*& p)
+{
+    uint32_t o = 0;
+    asm volatile("" : "+v"(o));
+    p += o;
+}
+
+// Keeps the computation of a value where it stands: without it the compiler
+// moves arithmetic down to the (later, guarded) code that uses its result,
+// and with it the lifetime of every operand.
+template <typename R>
+__device__ __forceinline__ void pin(cpx<R>& v)
+{
+    asm volatile("" : "+v"(v.x), "+v"(v.y));
+}
+
+// Radices of a wave-local transform of N over TP threads: two stages (b == 1)
+// or three, each radix a divisor of E = N / TP, or (the middle one) one whose
+// N / b butterflies divide evenly over the TP threads, so no lane idles.
+struct WPlan {
+    int a, b, c;
+};
+
+__host__ __device__ constexpr bool wave_radix(int r)
+{
+    return r == 2 || r == 3 || r == 4 || r == 5 || r == 6 || r == 8 || r == 10 || r == 12 || r == 16;
+}
+
+__host__ __device__ constexpr WPlan wave_plan(int N, int TP)
+{
+    const int E = N / TP;
+    WPlan best{0, 0, 0};
+    int score = 1 << 30;
+    for (int a = 2; a <= 16; ++a) {
+        if (!wave_radix(a) || E % a || N % a) continue;
+        for (int c = 2; c <= 16; ++c) {
+            if (!wave_radix(c) || E % c || (N / a) % c) continue;
+            const int b = N / a / c;
+            if (b == 1) {
+                // one exchange: the largest first radix
+                const int s = 100 - a;
+                if (s < score) { score = s; best = WPlan{a, 1, c}; }
+            } else if (wave_radix(b) && E % b == 0) {
+                // two exchanges: the most even radices
+                const int hi = a > b ? (a > c ? a : c) : (b > c ? b : c);
+                const int s = 1000 + 10 * hi + (16 - a);
+                if (s < score) { score = s; best = WPlan{a, b, c}; }
+            }
+        }
+    }
+    return best;
+}
+
+// --------------------------------------------------------------------------
+// Wave-local transform: the TP threads of a pencil are lanes t * CW + xl of
+// one wave (CW = 64 / TP columns side by side), thread t holding elements
+// n = t + TP e on entry and on return.  Exchange buffer: position pos of
+// column xl at slot (pos + pos / A) * CW + xl, A the first radix, so the
+// first stage's writes (stride A) and the later reads (stride 1) both spread
+// over the banks.  The twiddles lie in `tab` in the order in which the threads
+// read them (entry * TP + t).
+// --------------------------------------------------------------------------
+template <typename R, int N, int TP>
+struct WaveFft {
+    static constexpr int E = N / TP, CW = 64 / TP;
+    static constexpr WPlan P = wave_plan(N, TP);
+    static_assert(P.a > 0 && N % TP == 0 && 64 % TP == 0, "no wave-local plan");
+    static constexpr int A = P.a, B = P.b, C = P.c;
+    static constexpr int SLOTS = (N + N / A) * CW;
+    static constexpr int UB = E / B, UC = E / C;
+    static constexpr int TABB = B > 1 ? UB * (B - 1) * TP : 0;
+    static constexpr int NTAB = TABB + UC * (C - 1) * TP;
+
+    // the twiddle table, from the length-N roots
+    static __device__ __forceinline__ void fill(cpx<R>* tab, const cpx<R>* __restrict__ tw, int tid, int nt)
+    {
+        for (int i = tid; i < NTAB; i += nt) {
+            int n;
+            if (i < TABB) {
+                const int tt = i % TP, q = (i / TP) % (B > 1 ? B - 1 : 1) + 1, u = i / (TP * (B > 1 ? B - 1 : 1));
+                n = q * ((tt + TP * u) % A) * (N / (A * B));
+            } else {
+                const int k = i - TABB;
+                const int tt = k % TP, q = (k / TP) % (C - 1) + 1, u = k / (TP * (C - 1));
+                n = q * (tt + TP * u);
+            }
+            tab[i] = tw[n];
+        }
+    }
+
+    template <bool INV>
+    static __device__ __forceinline__ void run(cpx<R> (&v)[E], cpx<R>* lds, int t, int xl, const cpx<R>* tab)
+    {
+        constexpr int UA = E / A;
+        cpx<R>* const base = lds + xl;
+        const cpx<R>* tb = tab + t;
+        reread(tb);
+#pragma unroll
+        for (int u = 0; u < UA; ++u) {
+            cpx<R> a[A];
+#pragma unroll
+            for (int q = 0; q < A; ++q) a[q] = v[u + q * UA];
+            dft<R, INV, A, N>(a, nullptr);
+            cpx<R>* const o = base + (t + TP * u) * ((A + 1) * CW);
+#pragma unroll
+            for (int q = 0; q < A; ++q) o[q * CW] = a[q];
+        }
+        lds_sync<1>();
+        if constexpr (B > 1) {
+            cpx<R> a[UB][B];
+#pragma unroll
+            for (int u = 0; u < UB; ++u) {
+                const int j = t + TP * u;
+                const cpx<R>* const in = base + (j + j / A) * CW;
+#pragma unroll
+                for (int q = 0; q < B; ++q) a[u][q] = in[q * (N / B + N / B / A) * CW];
+            }
+            lds_sync<1>();
+#pragma unroll
+            for (int u = 0; u < UB; ++u) {
+                const int j = t + TP * u;
+                stage<INV, B>(a[u], tb + u * (B - 1) * TP);
+                cpx<R>* const o = base + ((j / A) * B * (A + 1) + j % A) * CW;
+#pragma unroll
+                for (int q = 0; q < B; ++q) o[q * (A + 1) * CW] = a[u][q];
+            }
+            lds_sync<1>();
+        }
+#pragma unroll
+        for (int u = 0; u < UC; ++u) {
+            const int j = t + TP * u;
+            const cpx<R>* const in = base + (j + j / A) * CW;
+            cpx<R> a[C];
+#pragma unroll
+            for (int q = 0; q < C; ++q) a[q] = in[q * (N / C + N / C / A) * CW];
+            stage<INV, C>(a, tb + TABB + u * (C - 1) * TP);
+#pragma unroll
+            for (int q = 0; q < C; ++q) v[u + q * UC] = a[q];
+        }
+        lds_sync<1>();   // the buffer is free for the next transform
+    }
+
+    // a[q] *= w[q] (q >= 1, w[q] at tb[(q - 1) TP]), then the radix-RAD butterfly
+    template <bool INV, int RAD>
+    static __device__ __forceinline__ void stage(cpx<R> (&a)[RAD], const cpx<R>* tb)
+    {
+        cpx<R> w[RAD];
+#pragma unroll
+        for (int q = 1; q < RAD; ++q) {
+            w[q] = tb[(q - 1) * TP];
+            if constexpr (!fused_tw<R, RAD>()) a[q] = INV ? cmulc(a[q], w[q]) : a[q] * w[q];
+        }
+        if constexpr (fused_tw<R, RAD>()) dft_tw<R, INV, RAD>(a, w);
+        else dft<R, INV, RAD, N>(a, nullptr);
+    }
+};
 
 }  // namespace gla

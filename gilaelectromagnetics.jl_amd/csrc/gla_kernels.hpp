@@ -776,6 +776,204 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_zpass(cpx<R>* __restrict__ W2
         }
 }
 
+// How a branch frequency k of axis 3 maps onto stored G^ entries for one
+// parity, without branches: entry k below f, m - k with the mirror sign
+// beyond (f past every k on an axis without mirror storage).
+struct ZMap {
+    int f, m;
+};
+
+__device__ __forceinline__ ZMap z_map(const AxisMap& a, int p)
+{
+    ZMap z;
+    z.f = a.sym ? (p ? a.fo : a.fe) : a.B;
+    z.m = p ? a.B - 1 : a.B;
+    return z;
+}
+
+// --------------------------------------------------------------------------
+// Pass 3, wave form: the same operation with every pencil inside one wave and
+// the two axis-3 parities on two waves of the workgroup.  A wave carries CW =
+// 64 / TP columns, TP threads each, and one parity: E = N / TP elements of
+// the three components are its whole state, and its exchanges are wave-local
+// (no workgroup barrier) through one LDS buffer of one component.  The
+// parities meet once, at the merge: each wave hands half of its results to
+// the other through LDS and stores the rows it keeps.  NG column groups fill
+// 128-byte rows (64-byte rows cost a quarter of the memory rate).  Bound by
+// the latency of the column's and G^'s loads at two or three waves per SIMD
+// (96^3, 16 right-hand sides: 62 us each for 253 MB).
+// --------------------------------------------------------------------------
+template <typename R, int N, int TP, int NG, int MODE, int MINW, int GD>
+__global__ __launch_bounds__(128 * NG, MINW) void k_zwave(cpx<R>* __restrict__ W2, int L1, int L2, int S3, int T3,
+                                                   int Z, int64_t w2s, const cpx<R>* __restrict__ gf,
+                                                   AxisMap a1, AxisMap a2, AxisMap a3,
+                                                   const cpx<R>* __restrict__ phz,
+                                                   const cpx<R>* __restrict__ tw,
+                                                   const int* __restrict__ order, int per_xcd, int nrhs)
+{
+    using F = WaveFft<R, N, TP>;
+    constexpr int E = N / TP, CW = 64 / TP, PX = CW * NG;
+    constexpr int H = (E + 1) / 2;             // rows wave 0 keeps
+    constexpr int SLW = F::SLOTS > 2 * H * 64 ? F::SLOTS : 2 * H * 64;
+    __shared__ cpx<R> lds[2 * NG][SLW];
+    __shared__ cpx<R> tab[F::NTAB + N];
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int p3 = wv & 1, grp = wv >> 1;
+    const int xl = lane % CW, t = lane / CW;
+    // workgroup -> (tile, right-hand side) as k_zpass
+    const int h = blockIdx.x;
+    const int q = h / 8;
+    const int l = (h % 8) * per_xcd + q / nrhs;
+    const int rhs = q % nrhs;
+    const int tile = order[l];
+    if (tile < 0) return;   // padding entry (whole workgroup)
+    const int c0 = (tile & 0xffff) * PX + grp * CW;
+    const int m1 = c0 + xl;
+    const int m2 = tile >> 16;
+    const bool act = m1 < L1;
+    const bool full = c0 + CW <= L1;
+    const int64_t cs = (int64_t)Z * L2 * L1;      // component stride
+    const int64_t zs = (int64_t)L2 * L1;
+    cpx<R>* const wgc = W2 + (int64_t)rhs * w2s + (int64_t)m2 * L1 + c0;
+    const uint32_t lob = ((uint32_t)xl + (uint32_t)t * (uint32_t)zs) * (uint32_t)sizeof(cpx<R>);
+    auto cp = [&](int c, int k) -> cpx<R>* {
+        return reinterpret_cast<cpx<R>*>(reinterpret_cast<char*>(wgc + ((int64_t)c * cs + (int64_t)k * zs)) + lob);
+    };
+    // the tables before the column: their wait does not cover the column's loads
+    F::fill(tab, tw, threadIdx.x, 128 * NG);
+    for (int i = threadIdx.x; i < N; i += 128 * NG) tab[F::NTAB + i] = phz[i];
+    __syncthreads();
+    cpx<R> w[3][E];
+    if (full && S3 >= N) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int e = 0; e < E; ++e) w[c][e] = *cp(c, TP * e);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                w[c][e] = (act && t + TP * e < S3) ? *cp(c, TP * e) : cpx<R>{R(0), R(0)};
+    }
+    const int p1 = m1 >= a1.B ? 1 : 0, k1 = m1 - p1 * a1.B;
+    const int p2 = m2 >= a2.B ? 1 : 0, k2 = m2 - p2 * a2.B;
+    int j1, s1, j2, s2;
+    axis_lookup(a1, act ? p1 : 0, act ? k1 : 0, j1, s1);
+    axis_lookup(a2, p2, k2, j2, s2);
+    const int uu = a1.U * a2.U;
+    const ZMap zm = z_map(a3, p3);
+    const cpx<R>* const gb =
+        gf + ((int64_t)((act ? p1 << 2 : 0) | (p2 << 1) | p3) * a3.U * uu + (j2 * a1.U + j1)) * 6;
+    if constexpr (MODE == 1) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const cpx<R> b = (act && t + TP * e + N < S3) ? *cp(c, TP * e + N) : cpx<R>{R(0), R(0)};
+                w[c][e] = p3 ? w[c][e] - b : w[c][e] + b;
+            }
+    }
+    const cpx<R>* const phl = tab + F::NTAB + t;
+    if (p3) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const cpx<R> ph = phl[TP * e];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) w[c][e] = ph * w[c][e];
+        }
+    }
+    cpx<R>* const mine = lds[wv];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) F::template run<false>(w[c], mine, t, xl, tab);
+    // symmetric 3x3 product, the loads of point e + 1 issued before point e
+    // is multiplied
+    {
+        const R f1 = R(s1), f2 = R(s2), s12 = R(s1 * s2);
+        cpx<R> gv[GD][6];
+        R sv[GD];
+        auto fetch = [&](int e, cpx<R>(&d)[6], R& sg) {
+            const int k = t + TP * e;
+            const bool low = k < zm.f;
+            sg = low ? R(1) : R(-1);
+            const cpx<R>* const g = gb + (int64_t)((low ? k : zm.m - k) * uu) * 6;
+#pragma unroll
+            for (int i = 0; i < 6; ++i) d[i] = g[i];
+        };
+#pragma unroll
+        for (int e = 0; e < GD && e < E; ++e) fetch(e, gv[e], sv[e]);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            cpx<R>(&g)[6] = gv[e % GD];
+            const R s13 = f1 * sv[e % GD], s23 = f2 * sv[e % GD];
+            const cpx<R> gxx = g[0], gyy = g[1], gzz = g[2];
+            const cpx<R> gxy = s12 * g[3], gxz = s13 * g[4], gyz = s23 * g[5];
+            const cpx<R> x0 = w[0][e], x1 = w[1][e], x2 = w[2][e];
+            w[0][e] = gxx * x0 + gxy * x1 + gxz * x2;
+            w[1][e] = gxy * x0 + gyy * x1 + gyz * x2;
+            w[2][e] = gxz * x0 + gyz * x1 + gzz * x2;
+            pin(w[0][e]);
+            pin(w[1][e]);
+            pin(w[2][e]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (e + GD < E) {
+                fetch(e + GD, gv[e % GD], sv[e % GD]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) F::template run<true>(w[c], mine, t, xl, tab);
+    if (p3) {
+        const cpx<R>* ph1 = phl;
+        reread(ph1);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const cpx<R> ph = ph1[TP * e];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) w[c][e] = cmulc(w[c][e], ph);
+        }
+    }
+    // merge: wave 0 keeps rows e < H, wave 1 the others; what a wave gives
+    // away goes through its own buffer, two halves of it in turn, so one
+    // barrier per component orders writes, reads and the next writes
+    const cpx<R>* const his = lds[wv ^ 1];
+    const int top = T3 < N ? T3 : N;
+    const bool all = full && T3 >= N;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const int o = (c & 1) * H * 64 + lane;
+        if (p3) {
+#pragma unroll
+            for (int e = 0; e < H; ++e) mine[o + e * 64] = w[c][e];
+        } else {
+#pragma unroll
+            for (int e = H; e < E; ++e) mine[o + (e - H) * 64] = w[c][e];
+        }
+        __syncthreads();
+        if (p3) {
+#pragma unroll
+            for (int e = H; e < E; ++e) {
+                const cpx<R> ev = his[o + (e - H) * 64];
+                const int n = t + TP * e;
+                if (all || (act && n < top)) *cp(c, TP * e) = ev + w[c][e];
+                if constexpr (MODE == 2)
+                    if (act && n + N < T3) *cp(c, TP * e + N) = ev - w[c][e];
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < H; ++e) {
+                const cpx<R> po = his[o + e * 64];
+                const int n = t + TP * e;
+                if (all || (act && n < top)) *cp(c, TP * e) = w[c][e] + po;
+                if constexpr (MODE == 2)
+                    if (act && n + N < T3) *cp(c, TP * e + N) = w[c][e] - po;
+            }
+        }
+    }
+}
+
 // --------------------------------------------------------------------------
 // Pass 3 of a partitioned operator: for target partition tp,
 //   Wo[tp] = IDFT_3( sum_s G^_{s,tp} DFT_3(W2[s]) ),

@@ -52,7 +52,7 @@ template <typename R, int N, int SMALL>
 struct ZK {
     static constexpr int CB = (int)sizeof(cpx<R>);
     static constexpr int POL = ptune(CB, N);
-    static constexpr int PXZ = ztune(CB, N, SMALL != 0).px;
+    static constexpr int PXZ = ztile(CB, N, SMALL != 0);
     static constexpr int TP_Z = N / pick_e(N, ztune(CB, N, SMALL != 0).e, 1024 / PXZ, GLA_ZWAVE != 0, POL);
     // pass 3 keeps each pencil inside one wave when its threads divide 64
     static constexpr int WL_Z = (GLA_ZWAVE != 0 && 64 % TP_Z == 0 && (TP_Z * PXZ) % 64 == 0) ? 1 : 0;
@@ -161,6 +161,23 @@ static hipError_t launch_zpass_shape(const Geom& g, const DevTab& tb, void* W2, 
     return hipGetLastError();
 }
 
+template <typename R, int N>
+static hipError_t launch_zwave(const Geom& g, const DevTab& tb, void* W2, int nrhs, hipStream_t st)
+{
+    constexpr WShape W = wtune((int)sizeof(cpx<R>), N);
+    // a thread's column address is a 32-bit byte offset ((column + t * L1 * L2) elements)
+    if ((int64_t)W.tp * g.L[0] * g.L[1] * (int64_t)sizeof(cpx<R>) >= ((int64_t)1 << 32)) return hipErrorInvalidValue;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(8 * tb.zper_xcd * nrhs), dim3(128 * W.ng), 0, st, (cpx<R>*)W2, g.L[0], g.L[1],
+                           g.S[2], g.T[2], g.Z, g.w2s, (const cpx<R>*)tb.gf, tb.am[0], tb.am[1], tb.am[2],
+                           (const cpx<R>*)tb.phz[2], (const cpx<R>*)tb.tw[2], tb.zorder, tb.zper_xcd, nrhs);
+        return hipGetLastError();
+    };
+    if (g.S[2] > g.B[2]) return go(k_zwave<R, N, W.tp, W.ng, 1, W.minw, W.gd>);
+    if (g.T[2] > g.B[2]) return go(k_zwave<R, N, W.tp, W.ng, 2, W.minw, W.gd>);
+    return go(k_zwave<R, N, W.tp, W.ng, 0, W.minw, W.gd>);
+}
+
 // pass 3 over nrhs right-hand sides: one launch has 8 * per_xcd workgroups per
 // right-hand side, so large batches are split to keep the grid within 2^31 - 1
 template <typename R, int N>
@@ -172,9 +189,13 @@ static hipError_t launch_zpass(const Geom& g, const DevTab& tb, void* W2, int nr
     for (int r0 = 0; r0 < nrhs; r0 += maxr) {
         const int cnt = nrhs - r0 < maxr ? nrhs - r0 : maxr;
         cpx<R>* const w = (cpx<R>*)W2 + (int64_t)r0 * g.w2s;
-        const bool small = (int64_t)g.L[0] * g.L[1] < ZSMALL_COLS;
-        const hipError_t e = small ? launch_zpass_shape<R, N, 1>(g, tb, w, cnt, st)
-                                   : launch_zpass_shape<R, N, 0>(g, tb, w, cnt, st);
+        hipError_t e;
+        if constexpr (wtune((int)sizeof(cpx<R>), N).tp > 0) {
+            e = launch_zwave<R, N>(g, tb, w, cnt, st);
+        } else {
+            const bool small = (int64_t)g.L[0] * g.L[1] < ZSMALL_COLS;
+            e = small ? launch_zpass_shape<R, N, 1>(g, tb, w, cnt, st) : launch_zpass_shape<R, N, 0>(g, tb, w, cnt, st);
+        }
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

@@ -133,6 +133,37 @@ constexpr ZShape ztune(int complex_bytes, int n, bool small)
     return small ? ztune_small(complex_bytes, n) : ztune_large(complex_bytes, n);
 }
 
+// pass 3, wave form (k_zwave): threads per pencil, column groups of 64 / tp
+// columns per workgroup, waves per SIMD asked of the compiler and G^ points in
+// flight; tp 0: the length runs k_zpass.  Taken where k_zpass's plan wastes
+// lanes or exchanges (96 = 4 6 4 against 4 3 2 4; 160, 192): us of pass 3,
+// k_zpass / k_zwave: 16 right-hand sides of 96^3 1113 / 999, 96^3 65.3 / 63.1,
+// 160^3 458 / 370, 192^3 716 / 638; not where it does not (128^3 153 / 179,
+// 64^3 22.2 / 21.4, 80^3 41.5 / 52.2, 96^3 ComplexF64 140 / 150).
+struct WShape {
+    int tp, ng, minw, gd;
+};
+
+constexpr WShape wtune(int complex_bytes, int n)
+{
+    if (complex_bytes == 8) {
+        switch (n) {
+            case 96: return {8, 2, 2, 2};
+            case 160: return {8, 2, 2, 2};
+            case 192: return {8, 2, 2, 2};
+            default: return {0, 0, 0, 0};
+        }
+    }
+    return {0, 0, 0, 0};
+}
+
+// columns per workgroup of pass 3, whichever kernel the length runs
+constexpr int ztile(int complex_bytes, int n, bool small)
+{
+    const WShape w = wtune(complex_bytes, n);
+    return w.tp > 0 ? 64 / w.tp * w.ng : ztune(complex_bytes, n, small).px;
+}
+
 constexpr RShape rtune(int complex_bytes, int n)
 {
     if (complex_bytes == 8) {
