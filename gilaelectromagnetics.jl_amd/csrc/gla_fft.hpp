@@ -52,6 +52,24 @@ __device__ __forceinline__ cpx<R> mul_mi(cpx<R> a)
     return {a.y, -a.x};
 }
 
+// A load or store of work planes; ONCE marks it as one whose line is not needed
+// again (streams() in gla_launch.hpp says where that pays).
+template <bool ONCE, typename R>
+__device__ __forceinline__ cpx<R> ld(const cpx<R>* p)
+{
+    if constexpr (!ONCE) return *p;
+    typedef R v2 __attribute__((ext_vector_type(2), aligned(sizeof(R))));
+    const v2 q = __builtin_nontemporal_load(reinterpret_cast<const v2*>(p));
+    return {q.x, q.y};
+}
+template <bool ONCE, typename R>
+__device__ __forceinline__ void st(cpx<R>* p, cpx<R> v)
+{
+    typedef R v2 __attribute__((ext_vector_type(2), aligned(sizeof(R))));
+    if constexpr (ONCE) __builtin_nontemporal_store(v2{v.x, v.y}, reinterpret_cast<v2*>(p));
+    else *p = v;
+}
+
 // ---------------------------------------------------------------------------
 // compile-time radix plan
 // ---------------------------------------------------------------------------

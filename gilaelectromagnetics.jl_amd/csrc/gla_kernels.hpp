@@ -206,7 +206,7 @@ constexpr int xk_of()
 // --------------------------------------------------------------------------
 // Pass 1: x-forward on contiguous rows.  One pencil = one (i2,i3,c) row of X.
 // --------------------------------------------------------------------------
-template <typename R, int N, int TP, int PEN, int MINW>
+template <typename R, int N, int TP, int PEN, int MINW, bool ONCE>
 __global__ __launch_bounds__(TP * PEN, MINW) void k_fwd_x(const cpx<R>* __restrict__ X, cpx<R>* __restrict__ W1,
                                                           int S1, int S2, int S3, int Y1, int Z,
                                                           int64_t xs, int64_t ws,
@@ -246,8 +246,8 @@ __global__ __launch_bounds__(TP * PEN, MINW) void k_fwd_x(const cpx<R>* __restri
     for (int e = 0; e < E; ++e) {
         const int n = t + TP * e;
         cpx<R> a = {R(0), R(0)}, b = {R(0), R(0)};
-        if (act && n < S1) a = xr[(int64_t)n * xd];
-        if (act && n + N < S1) b = xr[(int64_t)(n + N) * xd];
+        if (act && n < S1) a = ld<ONCE>(&xr[(int64_t)n * xd]);
+        if (act && n + N < S1) b = ld<ONCE>(&xr[(int64_t)(n + N) * xd]);
         v[0][e] = a + b;
         v[1][e] = phz[n] * (a - b);
     }
@@ -270,7 +270,7 @@ __global__ __launch_bounds__(TP * PEN, MINW) void k_fwd_x(const cpx<R>* __restri
 // --------------------------------------------------------------------------
 // Pass 5: x-inverse + merge/crop onto T1, optional y = alpha*res + beta*y.
 // --------------------------------------------------------------------------
-template <typename R, int N, int TP, int PEN, int MINW>
+template <typename R, int N, int TP, int PEN, int MINW, bool ONCE>
 __global__ __launch_bounds__(TP * PEN, MINW) void k_inv_x(const cpx<R>* __restrict__ W1, cpx<R>* __restrict__ Y,
                                                           int T1, int T2, int T3, int Y1, int Z,
                                                           int64_t ws, int64_t ys,
@@ -314,8 +314,8 @@ __global__ __launch_bounds__(TP * PEN, MINW) void k_inv_x(const cpx<R>* __restri
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int k = t + TP * e;
-        v[0][e] = act ? wr[k] : cpx<R>{R(0), R(0)};
-        v[1][e] = act ? wr[N + k] : cpx<R>{R(0), R(0)};
+        v[0][e] = act ? ld<ONCE>(&wr[k]) : cpx<R>{R(0), R(0)};
+        v[1][e] = act ? ld<ONCE>(&wr[N + k]) : cpx<R>{R(0), R(0)};
     }
     if constexpr (xk_of<R, N>() == 2) {
         PencilFft<R, N, TP, 1, PS, true, XSYNC, 2, PEN * PS, PADSH>::run(v, lds, t, pen, tw);
@@ -333,7 +333,7 @@ __global__ __launch_bounds__(TP * PEN, MINW) void k_inv_x(const cpx<R>* __restri
         const int64_t ny = (int64_t)n * yd;
         if (axpby == 1) r = alpha * r + (rd ? beta * yr[ny] : cpx<R>{R(0), R(0)});
         else if (axpby == 2) r = xr[n] - cr[n] * r;
-        yr[ny] = r;
+        st<ONCE>(&yr[ny], r);
     };
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -347,7 +347,7 @@ __global__ __launch_bounds__(TP * PEN, MINW) void k_inv_x(const cpx<R>* __restri
 // --------------------------------------------------------------------------
 // Pass 2: y-forward on bundles of PX consecutive axis-1 columns.
 // --------------------------------------------------------------------------
-template <typename R, int N, int TP, int PX, int MINW>
+template <typename R, int N, int TP, int PX, int MINW, bool ONCE>
 __global__ __launch_bounds__(TP * PX, MINW) void k_fwd_y(const cpx<R>* __restrict__ W1, cpx<R>* __restrict__ W2,
                                                    int L1, int S2, int S3, int Y1, int Z, int64_t w1s,
                                                    int64_t w2s, const cpx<R>* __restrict__ phz,
@@ -377,12 +377,12 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_fwd_y(const cpx<R>* __restric
     // whole bundle inside L1 and S2 >= N: the first-half loads need no guards
     if ((int)blockIdx.x * PX + PX <= L1 && S2 >= N) {
 #pragma unroll
-        for (int e = 0; e < E; ++e) v[0][e] = *sp(TP * e);
+        for (int e = 0; e < E; ++e) v[0][e] = ld<ONCE>(sp(TP * e));
     } else {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const int n = t + TP * e;
-            v[0][e] = (act && n < S2) ? *sp(TP * e) : cpx<R>{R(0), R(0)};
+            v[0][e] = (act && n < S2) ? ld<ONCE>(sp(TP * e)) : cpx<R>{R(0), R(0)};
         }
     }
 #pragma unroll
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_fwd_y(const cpx<R>* __restric
         const int n = t + TP * e;
         const cpx<R> a = v[0][e];
         cpx<R> b = {R(0), R(0)};
-        if (act && n + N < S2) b = *sp(TP * e + N);
+        if (act && n + N < S2) b = ld<ONCE>(sp(TP * e + N));
         v[0][e] = a + b;
         v[1][e] = phz[n] * (a - b);
     }
@@ -403,8 +403,8 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_fwd_y(const cpx<R>* __restric
     if (act) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            *dp(TP * e) = v[0][e];
-            *dp(N + TP * e) = v[1][e];
+            st<ONCE>(dp(TP * e), v[0][e]);
+            st<ONCE>(dp(N + TP * e), v[1][e]);
         }
     }
 }
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_fwd_y(const cpx<R>* __restric
 // --------------------------------------------------------------------------
 // Pass 4: y-inverse + merge/crop onto T2.
 // --------------------------------------------------------------------------
-template <typename R, int N, int TP, int PX, int MINW>
+template <typename R, int N, int TP, int PX, int MINW, bool ONCE>
 __global__ __launch_bounds__(TP * PX, MINW) void k_inv_y(const cpx<R>* __restrict__ W2, cpx<R>* __restrict__ W1,
                                                    int L1, int T2, int T3, int Y1, int Z, int64_t w2s,
                                                    int64_t w1s, const cpx<R>* __restrict__ phz,
@@ -443,14 +443,14 @@ __global__ __launch_bounds__(TP * PX, MINW) void k_inv_y(const cpx<R>* __restric
     if ((int)blockIdx.x * PX + PX <= L1) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            v[0][e] = *sp(TP * e);
-            v[1][e] = *sp(N + TP * e);
+            v[0][e] = ld<ONCE>(sp(TP * e));
+            v[1][e] = ld<ONCE>(sp(N + TP * e));
         }
     } else {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            v[0][e] = act ? *sp(TP * e) : cpx<R>{R(0), R(0)};
-            v[1][e] = act ? *sp(N + TP * e) : cpx<R>{R(0), R(0)};
+            v[0][e] = act ? ld<ONCE>(sp(TP * e)) : cpx<R>{R(0), R(0)};
+            v[1][e] = act ? ld<ONCE>(sp(N + TP * e)) : cpx<R>{R(0), R(0)};
         }
     }
     if constexpr (yk_of<R, N>() == 2) {

@@ -65,6 +65,21 @@ struct Epi {
     int64_t chis = 0;
 };
 
+// Whether passes 1, 2, 4 and 5 mark what they read once, and the results of
+// passes 2 and 5, as not needed again (ld / st of gla_fft.hpp): planes of
+// `bytes` no longer stay in the 256 MB last-level cache from pass to pass, and
+// marked they stop displacing what is read again (G^, the rest of the planes).
+// The line is 3/4 of that cache.  Without -> with, us a matvec:
+//   302 MB  128^3 ComplexF32 320 -> 298       226 MB  128x128x96 250 -> 233
+//   604 MB  128^3 ComplexF64 622 -> 576       254 MB  96^3, 2 at once 278 -> 261
+//   127 MB  96^3 136 -> 150                   147 MB  80^3 ComplexF64 171 -> 177
+//   plane kernels (W2 alone): 201 MB  64^3 ComplexF64, 4 at once 255 -> 235;
+//   151 MB  64x64x48, 8 at once 186 -> 202
+// (151 to 191 MB of W1 + W2: 3 to 5% either way).  Stores of passes 1 and 4,
+// and pass 3, gain nothing from it.
+constexpr int64_t STREAM_BYTES = 192 << 20;
+inline bool streams(int64_t bytes) { return bytes >= STREAM_BYTES; }
+
 bool len_supported(int n);
 bool len_fast(int n);             // 2^a x {1, 3, 5}: the lengths operators from geometry embed into
 int len_next_supported(int n);   // smallest fast length >= n, or 0

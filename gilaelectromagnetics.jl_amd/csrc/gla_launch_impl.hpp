@@ -94,8 +94,11 @@ static hipError_t launch_fwd_x(const Geom& g, const DevTab& tb, const void* X, v
 {
     using K = LenK<R, N>;
     const int rows = g.S[1] * g.S[2] * 3;
+    const auto kernel = streams((g.w1s + g.w2s) * nrhs * g.xp.np * K::CB)
+                            ? k_fwd_x<R, N, K::TP_ROW, K::PEN, 1, true>
+                            : k_fwd_x<R, N, K::TP_ROW, K::PEN, 1, false>;
     dim3 grid((rows + K::PEN - 1) / K::PEN, nrhs * g.xp.np);
-    hipLaunchKernelGGL((k_fwd_x<R, N, K::TP_ROW, K::PEN, 1>), grid, dim3(K::TP_ROW * K::PEN), 0, st,
+    hipLaunchKernelGGL(kernel, grid, dim3(K::TP_ROW * K::PEN), 0, st,
                        (const cpx<R>*)X, (cpx<R>*)W1, g.S[0], g.S[1], g.S[2], g.Y1, g.Z, g.xs, g.w1s,
                        (const cpx<R>*)tb.phz[0], (const cpx<R>*)tb.tw[0], g.xp);
     return hipGetLastError();
@@ -107,8 +110,11 @@ static hipError_t launch_inv_x(const Geom& g, const DevTab& tb, const void* W1, 
 {
     using K = LenK<R, N>;
     const int rows = g.T[1] * g.T[2] * 3;
+    const auto kernel = streams((g.w1s + g.w2s) * nrhs * g.yp.np * K::CB)
+                            ? k_inv_x<R, N, K::TP_ROW, K::PEN, 1, true>
+                            : k_inv_x<R, N, K::TP_ROW, K::PEN, 1, false>;
     dim3 grid((rows + K::PEN - 1) / K::PEN, nrhs * g.yp.np);
-    hipLaunchKernelGGL((k_inv_x<R, N, K::TP_ROW, K::PEN, 1>), grid, dim3(K::TP_ROW * K::PEN), 0, st,
+    hipLaunchKernelGGL(kernel, grid, dim3(K::TP_ROW * K::PEN), 0, st,
                        (const cpx<R>*)W1, (cpx<R>*)Y, g.T[0], g.T[1], g.T[2], g.Y1, g.Z, g.w1s, g.ys,
                        (const cpx<R>*)tb.phz[0], (const cpx<R>*)tb.tw[0], al, be, axpby,
                        (const cpx<R>*)epi.x, epi.xs, (const cpx<R>*)epi.chi, epi.chis, g.yp);
@@ -120,8 +126,11 @@ static hipError_t launch_fwd_y(const Geom& g, const DevTab& tb, const void* W1, 
 {
     using K = LenK<R, N>;
     constexpr int PX = K::PXY;
+    const auto kernel = streams((g.w1s + g.w2s) * nrhs * K::CB)
+                            ? k_fwd_y<R, N, K::TP_Y, PX, 1, true>
+                            : k_fwd_y<R, N, K::TP_Y, PX, 1, false>;
     dim3 grid((g.L[0] + PX - 1) / PX, g.S[2] * 3, nrhs);
-    hipLaunchKernelGGL((k_fwd_y<R, N, K::TP_Y, PX, 1>), grid, dim3(K::TP_Y * PX), 0, st, (const cpx<R>*)W1,
+    hipLaunchKernelGGL(kernel, grid, dim3(K::TP_Y * PX), 0, st, (const cpx<R>*)W1,
                        (cpx<R>*)W2, g.L[0], g.S[1], g.S[2], g.Y1, g.Z, g.w1s, g.w2s,
                        (const cpx<R>*)tb.phz[1], (const cpx<R>*)tb.tw[1]);
     return hipGetLastError();
@@ -132,8 +141,11 @@ static hipError_t launch_inv_y(const Geom& g, const DevTab& tb, const void* W2, 
 {
     using K = LenK<R, N>;
     constexpr int PX = K::PXY;
+    const auto kernel = streams((g.w1s + g.w2s) * nrhs * K::CB)
+                            ? k_inv_y<R, N, K::TP_Y, PX, 1, true>
+                            : k_inv_y<R, N, K::TP_Y, PX, 1, false>;
     dim3 grid((g.L[0] + PX - 1) / PX, g.T[2] * 3, nrhs);
-    hipLaunchKernelGGL((k_inv_y<R, N, K::TP_Y, PX, 1>), grid, dim3(K::TP_Y * PX), 0, st, (const cpx<R>*)W2,
+    hipLaunchKernelGGL(kernel, grid, dim3(K::TP_Y * PX), 0, st, (const cpx<R>*)W2,
                        (cpx<R>*)W1, g.L[0], g.T[1], g.T[2], g.Y1, g.Z, g.w2s, g.w1s,
                        (const cpx<R>*)tb.phz[1], (const cpx<R>*)tb.tw[1]);
     return hipGetLastError();

@@ -45,7 +45,7 @@ struct PlaneK {
 // = blockIdx.x of slot blockIdx.z.  plane[i2 N1 + m1]: rows are transformed
 // in place (wave-local), then each column's slots are its exchange buffer.
 // --------------------------------------------------------------------------
-template <typename R, int N1, int N2>
+template <typename R, int N1, int N2, bool ONCE>
 __global__ __launch_bounds__((PlaneK<R, N1, N2>::NTF)) void k_fwd_xy(
     const cpx<R>* __restrict__ X, cpx<R>* __restrict__ W2, int S1, int S2, int S3, int Z, int64_t xs, int64_t w2s,
     const cpx<R>* __restrict__ phz1, const cpx<R>* __restrict__ tw1, const cpx<R>* __restrict__ phz2,
@@ -125,7 +125,7 @@ __global__ __launch_bounds__((PlaneK<R, N1, N2>::NTF)) void k_fwd_xy(
 #pragma unroll
         for (int p = 0; p < 2; ++p)
 #pragma unroll
-            for (int e = 0; e < EY; ++e) w[(int64_t)(p * N2 + t + TPY * e) * (2 * N1) + m] = v[p][e];
+            for (int e = 0; e < EY; ++e) st<ONCE>(&w[(int64_t)(p * N2 + t + TPY * e) * (2 * N1) + m], v[p][e]);
     }
 }
 
@@ -133,7 +133,7 @@ __global__ __launch_bounds__((PlaneK<R, N1, N2>::NTF)) void k_fwd_xy(
 // Passes 4 + 5.  One workgroup: the plane (i3, c) = blockIdx.x of slot
 // blockIdx.y, both axis-1 parities (the merge needs them): plane[n2 2 N1 + m1].
 // --------------------------------------------------------------------------
-template <typename R, int N1, int N2>
+template <typename R, int N1, int N2, bool ONCE>
 __global__ __launch_bounds__((PlaneK<R, N1, N2>::NTI)) void k_inv_yx(
     const cpx<R>* __restrict__ W2, cpx<R>* __restrict__ Y, int T1, int T2, int T3, int Z, int64_t w2s, int64_t ys,
     const cpx<R>* __restrict__ phz1, const cpx<R>* __restrict__ tw1, const cpx<R>* __restrict__ phz2,
@@ -157,7 +157,7 @@ __global__ __launch_bounds__((PlaneK<R, N1, N2>::NTI)) void k_inv_yx(
 #pragma unroll
             for (int p = 0; p < 2; ++p)
 #pragma unroll
-                for (int e = 0; e < EY; ++e) v[p][e] = w[(int64_t)(p * N2 + t + TPY * e) * L1 + m];
+                for (int e = 0; e < EY; ++e) v[p][e] = ld<ONCE>(&w[(int64_t)(p * N2 + t + TPY * e) * L1 + m]);
         };
         load(xl);   // on its way while the tables are staged
         for (int i = threadIdx.x; i < N1; i += NT) {
@@ -210,7 +210,7 @@ __global__ __launch_bounds__((PlaneK<R, N1, N2>::NTI)) void k_inv_yx(
             if (axpby == 1) r = alpha * r + (rd ? beta * yr[ny] : cpx<R>{R(0), R(0)});
             else if (axpby == 2)
                 r = lsx[(int64_t)blockIdx.y * lsxs + row * T1 + n] - chi[(int64_t)blockIdx.y * chis + cell0 + n] * r;
-            yr[ny] = r;
+            st<ONCE>(&yr[ny], r);
         };
         const int top = T1 < N1 ? T1 : N1;
 #pragma unroll

@@ -19,7 +19,9 @@ static hipError_t plane_lds(K kernel, size_t lds)
 template <typename R, int N1, int N2>
 static hipError_t fwd_plane(const Geom& g, const DevTab& tb, const void* X, void* W2, int slots, hipStream_t st)
 {
-    const auto kernel = k_fwd_xy<R, N1, N2>;
+    const auto kernel = streams(g.w2s * slots * (int)sizeof(cpx<R>))
+                            ? k_fwd_xy<R, N1, N2, true>
+                            : k_fwd_xy<R, N1, N2, false>;
     const size_t lds = plane_bytes(g, (int)sizeof(cpx<R>), false);
     const hipError_t e = plane_lds(kernel, lds);
     if (e != hipSuccess) return e;
@@ -33,7 +35,9 @@ template <typename R, int N1, int N2>
 static hipError_t inv_plane(const Geom& g, const DevTab& tb, const void* W2, void* Y, int slots, cpx<R> al, cpx<R> be,
                             int axpby, const Epi& epi, hipStream_t st)
 {
-    const auto kernel = k_inv_yx<R, N1, N2>;
+    const auto kernel = streams(g.w2s * slots * (int)sizeof(cpx<R>))
+                            ? k_inv_yx<R, N1, N2, true>
+                            : k_inv_yx<R, N1, N2, false>;
     const size_t lds = plane_bytes(g, (int)sizeof(cpx<R>), true);
     const hipError_t e = plane_lds(kernel, lds);
     if (e != hipSuccess) return e;
