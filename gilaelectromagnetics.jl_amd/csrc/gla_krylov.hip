@@ -26,6 +26,9 @@ constexpr int KT = 256;          // threads per chunk workgroup
 constexpr int KW = KT / 64;      // waves per chunk workgroup
 constexpr int KG = 16;           // basis vectors per sweep over a chunk (2 KG sums, half a wave's lanes)
 
+// the sums' step, written out in FP64: the kernels' variants round alike
+__device__ __forceinline__ double fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 __device__ __forceinline__ double wave_sum(double v)
 {
 #pragma unroll
@@ -40,22 +43,44 @@ struct alignas(sizeof(cpx<R>) * VW) vec {
     cpx<R> e[VW];
 };
 
+// Bytes of basis that the last-level cache still holds between the products
+// and the update of one pass (192 MiB of its 256 MB).  A larger basis is read
+// with hints that its lines are not needed again -- in the products where more
+// than this follows, in the update, whose reads are a step's last, from twice
+// this on -- so that the rest of it, w and the matvec's planes stay.
+// 8 right-hand sides, 16 vectors of 3 x 64 x 64 x 48 ComplexF32 elements: the
+// products 117 -> 98 us, an Arnoldi step 490 -> 470; 2 x 20 vectors of
+// 6291456 ComplexF64: both 1627 -> 1500.  The update of half that basis, 302
+// MB, with the hint 66 -> 68, and products and update in turn 115 -> 125.
+constexpr int64_t KEEP_BYTES = 192 << 20;
+
+template <bool ONCE, typename V>
+__device__ __forceinline__ V load_vec(const V* p)
+{
+    if constexpr (ONCE) {
+        typedef uint32_t W __attribute__((ext_vector_type(sizeof(V) / 4), aligned(alignof(V))));
+        return __builtin_bit_cast(V, __builtin_nontemporal_load(reinterpret_cast<const W*>(p)));
+    } else {
+        return *p;
+    }
+}
+
 // one sweep over a chunk for G basis vectors i0 .. i0 + G - 1 (G = 0: the
 // norm of w alone).  Every load of a step (w and the G vectors) is issued
 // before the first use; a thread visits units of VW elements q = lo + VW t,
 // lo + VW (t + KT), ... in ascending order.  A last partial unit (n odd,
 // VW == 2) goes element by element.
-template <typename R, int G, int VW>
+template <typename R, int G, int VW, bool ONCE>
 __device__ __forceinline__ void dots_sweep(const cpx<R>* __restrict__ vp, int64_t vv, int i0,
                                            const cpx<R>* __restrict__ wp, int64_t lo, int64_t hi, bool first,
                                            double (&acc)[2 * KG + 1])
 {
     auto add = [&](const cpx<R>& b, const cpx<R>* a) {
-        if (first) acc[2 * KG] += (double)b.x * b.x + (double)b.y * b.y;
+        if (first) acc[2 * KG] = fma(b.x, b.x, fma(b.y, b.y, acc[2 * KG]));
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            acc[2 * g] += (double)a[g].x * b.x + (double)a[g].y * b.y;      // conj(a) b
-            acc[2 * g + 1] += (double)a[g].x * b.y - (double)a[g].y * b.x;
+            acc[2 * g] = fma(a[g].x, b.x, fma(a[g].y, b.y, acc[2 * g]));   // conj(a) b
+            acc[2 * g + 1] = fma(a[g].x, b.y, fma(-a[g].y, b.x, acc[2 * g + 1]));
         }
     };
     const cpx<R>* const v0 = vp + (int64_t)i0 * vv;
@@ -65,7 +90,7 @@ __device__ __forceinline__ void dots_sweep(const cpx<R>* __restrict__ vp, int64_
         const V b = *reinterpret_cast<const V*>(wp + q);
         V a[G > 0 ? G : 1];
 #pragma unroll
-        for (int g = 0; g < G; ++g) a[g] = *reinterpret_cast<const V*>(v0 + g * vv + q);
+        for (int g = 0; g < G; ++g) a[g] = load_vec<ONCE>(reinterpret_cast<const V*>(v0 + g * vv + q));
         __builtin_amdgcn_sched_barrier(0);   // keep the step's loads ahead of the arithmetic
 #pragma unroll
         for (int e = 0; e < VW; ++e) {
@@ -83,13 +108,13 @@ __device__ __forceinline__ void dots_sweep(const cpx<R>* __restrict__ vp, int64_
     }
 }
 
-template <typename R, int VW, int G>
+template <typename R, int VW, int G, bool ONCE>
 __device__ __forceinline__ void dots_count(int count, const cpx<R>* __restrict__ vp, int64_t vv, int i0,
                                            const cpx<R>* __restrict__ wp, int64_t lo, int64_t hi, bool first,
                                            double (&acc)[2 * KG + 1])
 {
-    if (count == G) dots_sweep<R, G, VW>(vp, vv, i0, wp, lo, hi, first, acc);
-    else if constexpr (G > 0) dots_count<R, VW, G - 1>(count, vp, vv, i0, wp, lo, hi, first, acc);
+    if (count == G) dots_sweep<R, G, VW, ONCE>(vp, vv, i0, wp, lo, hi, first, acc);
+    else if constexpr (G > 0) dots_count<R, VW, G - 1, ONCE>(count, vp, vv, i0, wp, lo, hi, first, acc);
 }
 
 // Block products of one chunk.  part layout: [r][slot][chunk]; slots 0..nv-1
@@ -99,7 +124,7 @@ __device__ __forceinline__ void dots_count(int count, const cpx<R>* __restrict__
 // TB/s where a bare read of the basis takes 97).  Before, with 8 vectors a
 // sweep, 8-byte loads, one wave sum per value and 4096-element chunks, it
 // took 129 us, and 8 x 98304 elements 34 us (now 21).
-template <typename R, int VW>
+template <typename R, int VW, bool LARGE>
 __global__ __launch_bounds__(KT) void k_dots(const cpx<R>* __restrict__ V, int64_t vr, int64_t vv,
                                              const cpx<R>* __restrict__ w, int64_t wr, int64_t n, int nv,
                                              const int64_t* __restrict__ ncol, int64_t chunk, int nchunk, int nslot,
@@ -110,6 +135,8 @@ __global__ __launch_bounds__(KT) void k_dots(const cpx<R>* __restrict__ V, int64
     const int nvr = ncol ? (int)(ncol[r] < 0 ? 0 : ncol[r] < nv ? ncol[r] : nv) : nv;
     const int64_t lo = (int64_t)c * chunk;
     const int64_t hi = lo + chunk < n ? lo + chunk : n;
+    // more basis behind this chunk than stays in the last-level cache
+    const bool once = LARGE && ((int64_t)(gridDim.y - r) * n - lo) * nv * (int64_t)sizeof(cpx<R>) > KEEP_BYTES;
     const cpx<R>* wp = w + r * wr;
     const cpx<R>* vp = V + r * vr;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -122,7 +149,8 @@ __global__ __launch_bounds__(KT) void k_dots(const cpx<R>* __restrict__ V, int64
         for (int g = 0; g < 2 * KG + 1; ++g) acc[g] = 0.0;
         const bool first = i0 == 0 && self;
         const int count = nvr - i0 < KG ? nvr - i0 : KG;
-        dots_count<R, VW, KG>(count, vp, vv, i0, wp, lo, hi, first, acc);
+        if (once) dots_count<R, VW, KG, LARGE>(count, vp, vv, i0, wp, lo, hi, first, acc);
+        else dots_count<R, VW, KG, false>(count, vp, vv, i0, wp, lo, hi, first, acc);
         // the wave's 2 KG sums, halving the values a lane carries at each step:
         // lane l ends with value l / 2 (37 exchanges where a sum per value
         // takes 192)
@@ -166,7 +194,7 @@ constexpr int KU = 4;
 // last to first: the products before it read the basis first to last, so the
 // end of it is still in the last-level cache (products and update of the
 // same case together: 264 us first to last, 231 last to first).
-template <typename R, int VW>
+template <typename R, int VW, bool ONCE>
 __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64_t vr, int64_t vv,
                                              const cpx<double>* __restrict__ h, int64_t hr,
                                              cpx<R>* __restrict__ w, int64_t wr, int64_t n, int nv,
@@ -185,8 +213,8 @@ __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64
     cpx<R>* wp = w + r * wr;
     double nrm = 0.0;
     auto finish = [&](cpx<R> o, double ar, double ai) {
-        const cpx<R> res{R((double)o.x + s * ar), R((double)o.y + s * ai)};
-        nrm += (double)res.x * res.x + (double)res.y * res.y;
+        const cpx<R> res{R(fma(s, ar, (double)o.x)), R(fma(s, ai, (double)o.y))};
+        nrm = fma(res.x, res.x, fma(res.y, res.y, nrm));
         return res;
     };
     const int64_t whole = lo + (hi - lo) / VW * VW;   // end of the whole units
@@ -207,8 +235,8 @@ __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64
         auto mac = [&](const cpx<double>& cc, int e, const U& a) {
 #pragma unroll
             for (int k = 0; k < VW; ++k) {
-                ar[e][k] += cc.x * a.e[k].x - cc.y * a.e[k].y;
-                ai[e][k] += cc.x * a.e[k].y + cc.y * a.e[k].x;
+                ar[e][k] = fma(cc.x, a.e[k].x, fma(-cc.y, a.e[k].y, ar[e][k]));
+                ai[e][k] = fma(cc.x, a.e[k].y, fma(cc.y, a.e[k].x, ai[e][k]));
             }
         };
         int i = 0;
@@ -218,7 +246,7 @@ __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64
             for (int u = 0; u < KU; ++u)
 #pragma unroll
                 for (int e = 0; e < E; ++e)
-                    a[u][e] = *reinterpret_cast<const U*>(vp + (int64_t)(i + u) * vv + qe[e]);
+                    a[u][e] = load_vec<ONCE>(reinterpret_cast<const U*>(vp + (int64_t)(i + u) * vv + qe[e]));
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int u = 0; u < KU; ++u) {
@@ -230,7 +258,7 @@ __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64
         for (; i < nv; ++i) {
             U a[E];
 #pragma unroll
-            for (int e = 0; e < E; ++e) a[e] = *reinterpret_cast<const U*>(vp + (int64_t)i * vv + qe[e]);
+            for (int e = 0; e < E; ++e) a[e] = load_vec<ONCE>(reinterpret_cast<const U*>(vp + (int64_t)i * vv + qe[e]));
             const cpx<double> cc = hp[i];
 #pragma unroll
             for (int e = 0; e < E; ++e) mac(cc, e, a[e]);
@@ -249,8 +277,8 @@ __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64
         for (int i = 0; i < nv; ++i) {
             const cpx<R> a = vp[(int64_t)i * vv + whole];
             const cpx<double> cc = hp[i];
-            ar += cc.x * a.x - cc.y * a.y;
-            ai += cc.x * a.y + cc.y * a.x;
+            ar = fma(cc.x, a.x, fma(-cc.y, a.y, ar));
+            ai = fma(cc.x, a.y, fma(cc.y, a.x, ai));
         }
         wp[whole] = finish(wp[whole], ar, ai);
     }
@@ -374,7 +402,11 @@ hipError_t run_krylov_dots(int64_t k, int nv, int64_t n, const void* V, int64_t 
     const int nchunk = (int)((n + chunk - 1) / chunk);
     const int self = w2 != nullptr;
     const int nslot = nv + 1;
-    const auto kernel = wide_ok<R>(V, vr, vv, w, wr) ? k_dots<R, sizeof(cpx<R>) == 8 ? 2 : 1> : k_dots<R, 1>;
+    const bool large = k * nv * n * (int64_t)sizeof(cpx<R>) > KEEP_BYTES;
+    const auto kernel = wide_ok<R>(V, vr, vv, w, wr)
+                            ? (large ? k_dots<R, sizeof(cpx<R>) == 8 ? 2 : 1, true>
+                                     : k_dots<R, sizeof(cpx<R>) == 8 ? 2 : 1, false>)
+                            : (large ? k_dots<R, 1, true> : k_dots<R, 1, false>);
     hipLaunchKernelGGL(kernel, dim3(nchunk, (unsigned)k), dim3(KT), 0, st, (const cpx<R>*)V, vr, vv,
                        (const cpx<R>*)w, wr, n, nv, ncol, chunk, nchunk, nslot, self, (double*)part);
     hipError_t e = hipGetLastError();
@@ -392,9 +424,11 @@ hipError_t run_krylov_axpy(int64_t k, int nv, int64_t n, const void* V, int64_t 
     const int64_t chunk = krylov_chunk(n);
     const int nchunk = (int)((n + chunk - 1) / chunk);
     const int norm = w2 != nullptr;
+    const bool large = k * nv * n * (int64_t)sizeof(cpx<R>) > 2 * KEEP_BYTES;
     const auto kernel = wide_ok<R>(nv > 0 ? V : w, nv > 0 ? vr : 0, nv > 0 ? vv : 0, w, wr)
-                            ? k_axpy<R, sizeof(cpx<R>) == 8 ? 2 : 1>
-                            : k_axpy<R, 1>;
+                            ? (large ? k_axpy<R, sizeof(cpx<R>) == 8 ? 2 : 1, true>
+                                     : k_axpy<R, sizeof(cpx<R>) == 8 ? 2 : 1, false>)
+                            : (large ? k_axpy<R, 1, true> : k_axpy<R, 1, false>);
     hipLaunchKernelGGL(kernel, dim3(nchunk, (unsigned)k), dim3(KT), 0, st, (const cpx<R>*)V, vr, vv,
                        (const cpx<double>*)h, hr, (cpx<R>*)w, wr, n, nv, ncol, s, chunk, nchunk, norm,
                        (double*)part);
