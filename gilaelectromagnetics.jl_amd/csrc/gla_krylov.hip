@@ -120,8 +120,8 @@ __device__ __forceinline__ void dots_count(int count, const cpx<R>* __restrict__
 // Block products of one chunk.  part layout: [r][slot][chunk]; slots 0..nv-1
 // the dots, slot nv the squared norm of w (when requested).  Bound by HBM:
 // each right-hand side's basis is read once (8 right-hand sides, 16 vectors
-// of 3 x 64 x 64 x 48 ComplexF32 elements, 640 MB: 111 us with its sums, 5.8
-// TB/s where a bare read of the basis takes 97).  Before, with 8 vectors a
+// of 3 x 64 x 64 x 48 ComplexF32 elements, 640 MB: 98 us with its sums, 6.1
+// TB/s, as fast as a bare read of the basis).  Before, with 8 vectors a
 // sweep, 8-byte loads, one wave sum per value and 4096-element chunks, it
 // took 129 us, and 8 x 98304 elements 34 us (now 21).
 template <typename R, int VW, bool LARGE>
@@ -193,7 +193,8 @@ constexpr int KU = 4;
 // ascending order (E units of VW elements at a time).  Right-hand sides run
 // last to first: the products before it read the basis first to last, so the
 // end of it is still in the last-level cache (products and update of the
-// same case together: 264 us first to last, 231 last to first).
+// same case together: 264 us first to last, 231 last to first, 224 with the
+// hints of KEEP_BYTES).
 template <typename R, int VW, bool ONCE>
 __global__ __launch_bounds__(KT) void k_axpy(const cpx<R>* __restrict__ V, int64_t vr, int64_t vv,
                                              const cpx<double>* __restrict__ h, int64_t hr,
