@@ -378,7 +378,7 @@ bool mirrored(const gla_dims& d, const std::vector<std::complex<double>>& fur, i
 // out, and mirror storage on the device: the longer circulant has the same
 // symmetry, so pass 3 reads half the G^ per such axis (self 100x60x44 on
 // (128,64,48), ComplexF32: 151 -> 21 MB of G^, pass 3 37 -> 20 us, the call
-// 110 -> 92 us).  Data read from a file is checked rather than trusted.
+// 110 -> 92 us).  Data handed in or read from a file are checked, not trusted.
 AxisStore axis_store(const gla_opr_s& h, const std::vector<std::complex<double>>& fur, int a, bool made)
 {
     const gla_dims& d = h.dims;
@@ -681,7 +681,7 @@ gla_status gla_opr_create_from_fur(const gla_opts* opts, const gla_vol* trg, con
     if ((s = dims_impl(&t2, sp, DIMS_EXACT, &d))) return s;
     bool same = true;
     for (int a = 0; a < 3; ++a) same = same && d.dev_brn[a] == ref.brn[a];
-    if (same) return create_common(opts, &t2, sp, d, fur, fur_dtype, fur_len, true, out);
+    if (same) return create_common(opts, &t2, sp, d, fur, fur_dtype, fur_len, false, out);
     // a branch length without a compiled transform: the data is re-expressed
     // at the next fast length (gla::refur) in FP64
     const int64_t Ut = ref.fur_ext[0] * ref.fur_ext[1] * ref.fur_ext[2];
@@ -701,15 +701,18 @@ gla_status gla_opr_create_from_fur(const gla_opts* opts, const gla_vol* trg, con
         DevGuard g(opts->device);
         if ((s = gla::refur(ref, d, furd, re, err))) return fail(s, err);
     }
-    return create_common(opts, &t2, sp, d, re.data(), GLA_C128, (int64_t)re.size(), true, out);
+    return create_common(opts, &t2, sp, d, re.data(), GLA_C128, (int64_t)re.size(), false, out);
 }
 
 }  // extern "C"
 
 namespace {
 
-// made: the branches come from this library's own setup or re-embedding, so
-// an embedded axis's mirror symmetry needs no check
+// made: the branches come from this library's own setup, so an embedded
+// axis's mirror symmetry needs no check.  Branches handed in do, re-embedded
+// ones too: the longer spectrum is its own mirror image only if their
+// self-image entries (frequency 0 and L / 2) of the components odd in the
+// axis vanish.
 gla_status create_common(const gla_opts* opts, const gla_vol* trg, const gla_vol* src, gla_dims d, const void* fur,
                          int32_t fur_dtype, int64_t fur_len, bool made, gla_opr_t* out)
 {
