@@ -343,17 +343,22 @@ struct AxisStore {
     bool sym;
 };
 
-// Whether the branches are their own mirror images along axis a up to
-// rounding, F(L - m) = s F(m) with s = -1 for the off-diagonal components
-// that involve the axis (the relation of a self axis).
-bool mirrored(const gla_dims& d, const std::vector<std::complex<double>>& fur, int a, double tol)
+// Whether the branches are their own mirror images along axis a, F(L - m) =
+// s F(m) with s = -1 for the off-diagonal components that involve the axis
+// (the relation of a self axis), up to rounding: of the stored entries (two
+// ComplexF32 neighbours, `rel` of the entry) and of the FP64 transforms that
+// made them (32 eps of the largest entry; 5e-16 of it measured on re-embedded
+// data, 6e-15 on branches from face integrals).  A looser bound would lose
+// components far below the largest entry.
+bool mirrored(const gla_dims& d, const std::vector<std::complex<double>>& fur, int a)
 {
     const int64_t U[3] = {d.fur_ext[0], d.fur_ext[1], d.fur_ext[2]};
     const int64_t Ut = U[0] * U[1] * U[2], B = U[a];
     const int64_t st = a == 0 ? 1 : a == 1 ? U[0] : U[0] * U[1];
     double top = 0;
     for (const auto& v : fur) top = std::max(top, std::max(std::fabs(v.real()), std::fabs(v.imag())));
-    const double lim = tol * top;
+    const double lim = 0x1p-47 * top, rel = d.dtype == GLA_C64 ? 0x1p-22 : 0.0;
+    auto differ = [=](double u, double v) { return std::fabs(v - u) > lim + rel * std::fabs(u); };
     static const int odd[3][2] = {{3, 4}, {3, 5}, {4, 5}};
     for (int b = 0; b < 8; ++b)
         for (int c = 0; c < 6; ++c) {
@@ -365,9 +370,7 @@ bool mirrored(const gla_dims& d, const std::vector<std::complex<double>>& fur, i
                     const int64_t m = p ? B - 1 - k : (B - k) % B;
                     const std::complex<double>*const u = f + lo + k * st, *const v = f + lo + m * st;
                     for (int64_t i = 0; i < st; ++i)
-                        if (std::fabs(v[i].real() - s * u[i].real()) > lim ||
-                            std::fabs(v[i].imag() - s * u[i].imag()) > lim)
-                            return false;
+                        if (differ(s * u[i].real(), v[i].real()) || differ(s * u[i].imag(), v[i].imag())) return false;
                 }
         }
     return true;
@@ -387,7 +390,7 @@ AxisStore axis_store(const gla_opr_s& h, const std::vector<std::complex<double>>
                       h.trg.org_num[a] * h.src.org_den[a] == h.src.org_num[a] * h.trg.org_den[a];
     const int B = (int)d.dev_brn[a];
     const bool half = same && d.dev_brn[a] != d.brn[a] && n_src_part(d) * n_trg_part(d) == 1 && B > 2 &&
-                      (made || mirrored(d, fur, a, d.dtype == GLA_C64 ? 1e-6 : 1e-12));
+                      (made || mirrored(d, fur, a));
     return half ? AxisStore{B / 2 + 1, true} : AxisStore{(int)d.fur_ext[a], false};
 }
 
