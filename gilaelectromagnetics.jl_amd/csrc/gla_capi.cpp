@@ -18,6 +18,7 @@
 #include "gla_launch.hpp"
 #include "gla_planes.hpp"
 #include "gla_setup.hpp"
+#include "gla_slots.hpp"
 
 namespace {
 
@@ -128,10 +129,8 @@ struct gla_opr_s {
     gla::DevTab tab{};
     std::shared_ptr<DevData> dev;
     std::shared_ptr<std::vector<char>> fur_host;   // reference layout, operator dtype
-    void* w1 = nullptr;
-    void* w2 = nullptr;
-    int64_t w1_slots = 0, w2_slots = 0;   // right-hand sides (times partitions) w1 / w2 hold
-    int batches = 0;   // recorded batches that use w1 / w2 (they must not move)
+    gla::WorkPlanes ws;
+    int batches = 0;   // recorded batches that use the work planes (they must not move)
     // device copies of the host arrays of gla_opr_apply_host (grown as
     // needed, kept until release), under their own lock
     void* hx = nullptr;
@@ -141,10 +140,10 @@ struct gla_opr_s {
     std::mutex mu;
     ~gla_opr_s()
     {
-        if (w1 || w2 || hx || hy) {
+        if (ws.w1 || ws.w2 || hx || hy) {
             DevGuard g(opts.device);
-            if (w1) (void)hipFree(w1);
-            if (w2) (void)hipFree(w2);
+            if (ws.w1) (void)hipFree(ws.w1);
+            if (ws.w2) (void)hipFree(ws.w2);
             if (hx) (void)hipFree(hx);
             if (hy) (void)hipFree(hy);
         }
@@ -512,31 +511,12 @@ void part_offset(int64_t p, const int64_t div[3], int o[3])
 
 size_t elem_bytes(int dtype) { return dtype == GLA_C64 ? 8 : 16; }
 
-// Work-plane slots of nrhs right-hand sides.  A partitioned operator takes all
-// partitions of a pass in one launch (run_matvec_parts: each source partition
-// transformed once, the sum over them between the transforms) when its slots
-// stay within kPartBytes; otherwise, or when only that much work memory is at
-// hand, it runs the five passes once per (source, target) pair on one slot
-// per right-hand side.  48^3 fine cells (8 source partitions) on 24^3 coarse
-// ones, ComplexF32: 211 us pair by pair (40 launches of too few workgroups
-// each, the forward and inverse transforms of pass 3 once per pair), 69 us in
-// five launches.  The bound is on memory: it keeps the work planes of one
-// call within a hundredth of the GPU's.
-constexpr int64_t kPartBytes = (int64_t)2 << 30;
+using gla::Slots;
 
-struct Slots {
-    int64_t w1, w2;
-};
-
-Slots pair_slots(int64_t nrhs) { return Slots{nrhs, nrhs}; }
-
-Slots part_slots(const gla_opr_s& h, int64_t nrhs)
+gla::SlotCost slot_cost(const gla_opr_s& h)
 {
-    const int64_t Ps = n_src_part(h.dims), Pt = n_trg_part(h.dims);
-    if (Ps * Pt == 1) return pair_slots(nrhs);
-    const Slots s{nrhs * std::max(Ps, Pt), nrhs * (Ps + (Pt > 1 ? Pt : 0))};
-    const int64_t bytes = (s.w1 * h.geom.w1s + s.w2 * h.geom.w2s) * (int64_t)elem_bytes(h.dims.dtype);
-    return s.w1 <= 65535 && bytes <= kPartBytes ? s : pair_slots(nrhs);
+    const int64_t eb = (int64_t)elem_bytes(h.dims.dtype);
+    return gla::SlotCost{n_src_part(h.dims), n_trg_part(h.dims), h.geom.w1s * eb, h.geom.w2s * eb};
 }
 
 // The whole matvec on `st` with work planes w1 / w2 of `have` slots.  Pair by
@@ -549,6 +529,7 @@ Slots part_slots(const gla_opr_s& h, int64_t nrhs)
 hipError_t matvec_all(const gla_opr_s& h, const void* x, void* y, void* w1, void* w2, Slots have, int nrhs, double ar,
                       double ai, double br, double bi, int axpby, const gla::Epi& epi, hipStream_t st)
 {
+    if (!gla::covers(have, gla::pair_slots(nrhs))) return hipErrorInvalidValue;
     const bool c64 = h.dims.dtype == GLA_C64;
     auto one = [&](const gla::Geom& g, const gla::DevTab& tb, double b_r, double b_i, int ax) {
         return c64 ? gla::run_matvec<float>(g, tb, x, y, w1, w2, nrhs, ar, ai, b_r, b_i, ax, epi, st)
@@ -558,8 +539,8 @@ hipError_t matvec_all(const gla_opr_s& h, const void* x, void* y, void* w1, void
     if (Ps * Pt == 1) return one(h.geom, h.tab, br, bi, axpby);
     if (axpby == 2) return hipErrorInvalidValue;   // self operators only, never partitioned
     const int64_t pair = 8 * h.dims.fur_ext[0] * h.dims.fur_ext[1] * h.dims.fur_ext[2] * 6;
-    const Slots s = part_slots(h, nrhs);
-    if (s.w1 > nrhs && have.w1 >= s.w1 && have.w2 >= s.w2)
+    const gla::SlotCost cost = slot_cost(h);
+    if (nrhs <= gla::part_limit(cost) && gla::covers(have, gla::part_slots(cost, nrhs)))
         return c64 ? gla::run_matvec_parts<float>(h.geom, h.tab, x, y, w1, w2, nrhs, (int)Ps, (int)Pt, pair, ar, ai, br,
                                                   bi, axpby, st)
                    : gla::run_matvec_parts<double>(h.geom, h.tab, x, y, w1, w2, nrhs, (int)Ps, (int)Pt, pair, ar, ai,
@@ -581,45 +562,33 @@ hipError_t matvec_all(const gla_opr_s& h, const void* x, void* y, void* w1, void
     return hipSuccess;
 }
 
-// Work buffers of nrhs right-hand sides (GLA_OK also when they cannot grow but
-// hold what the pair-by-pair form needs).
+// Work planes for nrhs right-hand sides (gla::ensure_planes).
 gla_status ensure_ws(gla_opr_t h, int64_t nrhs, bool may_grow = true)
 {
-    const Slots want = part_slots(*h, nrhs);
-    if (h->w1_slots >= want.w1 && h->w2_slots >= want.w2) return GLA_OK;
-    const bool fits = h->w1_slots >= nrhs && h->w2_slots >= nrhs;
-    if (fits && (!may_grow || h->batches > 0)) return GLA_OK;
-    if (!may_grow)
-        return fail(GLA_ERR_ARG, "work buffers for " + std::to_string(nrhs) +
-                                     " right-hand sides must be reserved (gla_opr_reserve) before capture");
-    if (h->batches > 0)
-        return fail(GLA_ERR_ARG, "the operator's work buffers are recorded in a batch; "
-                                 "destroy the batch before applying it to more right-hand sides");
-    const size_t eb = elem_bytes(h->dims.dtype);
-    if (h->w1) { (void)hipFree(h->w1); h->w1 = nullptr; }
-    if (h->w2) { (void)hipFree(h->w2); h->w2 = nullptr; }
-    h->w1_slots = h->w2_slots = 0;
-    auto grow = [&](Slots s) {
-        hipError_t e = hipMalloc(&h->w1, (size_t)(h->geom.w1s * s.w1) * eb);
-        if (e != hipSuccess) { h->w1 = nullptr; return e; }
-        e = hipMalloc(&h->w2, (size_t)(h->geom.w2s * s.w2) * eb);
-        if (e != hipSuccess) {
-            h->w2 = nullptr;
-            (void)hipFree(h->w1);
-            h->w1 = nullptr;
-            return e;
+    struct {
+        hipError_t err = hipSuccess;
+        void* alloc(int64_t bytes)
+        {
+            void* p = nullptr;
+            const hipError_t e = hipMalloc(&p, (size_t)bytes);
+            if (e == hipSuccess) return p;
+            err = e;
+            (void)hipGetLastError();
+            return nullptr;
         }
-        h->w1_slots = s.w1;
-        h->w2_slots = s.w2;
-        return e;
-    };
-    hipError_t e = grow(want);
-    if (e != hipSuccess && want.w1 > nrhs) {
-        (void)hipGetLastError();
-        e = grow(pair_slots(nrhs));
+        void release(void* p) { (void)hipFree(p); }
+    } mem;
+    switch (gla::ensure_planes(h->ws, slot_cost(*h), nrhs, may_grow, h->batches > 0, mem)) {
+        case gla::Ensure::ok: return GLA_OK;
+        case gla::Ensure::capture:
+            return fail(GLA_ERR_ARG, "work buffers for " + std::to_string(nrhs) +
+                                         " right-hand sides must be reserved (gla_opr_reserve) before capture");
+        case gla::Ensure::pinned:
+            return fail(GLA_ERR_ARG, "the operator's work buffers are recorded in a batch; "
+                                     "destroy the batch before applying it to more right-hand sides");
+        default:
+            return fail(GLA_ERR_HIP, std::string("hipMalloc of the work buffers: ") + hipGetErrorString(mem.err));
     }
-    if (e != hipSuccess) return fail(GLA_ERR_HIP, std::string("hipMalloc of the work buffers: ") + hipGetErrorString(e));
-    return GLA_OK;
 }
 
 gla_status run(gla_opr_t h, const void* x, int64_t nx, void* y, int64_t ny, int64_t nrhs, double ar,
@@ -637,13 +606,12 @@ gla_status run(gla_opr_t h, const void* x, int64_t nx, void* y, int64_t ny, int6
     // growing the work buffers frees and allocates, which a stream under
     // graph capture must not see
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const Slots want = part_slots(*h, nrhs);
-    const bool enough = h->w1_slots >= want.w1 && h->w2_slots >= want.w2;
-    const bool capturing = !enough && stream && hipStreamIsCapturing((hipStream_t)stream, &cs) == hipSuccess &&
+    const bool capturing = h->ws.nrhs < nrhs && stream &&
+                           hipStreamIsCapturing((hipStream_t)stream, &cs) == hipSuccess &&
                            cs != hipStreamCaptureStatusNone;
     gla_status s = ensure_ws(h, nrhs, !capturing);
     if (s) return s;
-    const hipError_t e = matvec_all(*h, x, y, h->w1, h->w2, Slots{h->w1_slots, h->w2_slots}, (int)nrhs, ar, ai, br, bi, axpby, epi,
+    const hipError_t e = matvec_all(*h, x, y, h->ws.w1, h->ws.w2, h->ws.held, (int)nrhs, ar, ai, br, bi, axpby, epi,
                                     (hipStream_t)stream);
     if (e != hipSuccess) return fail(GLA_ERR_HIP, std::string("matvec launch: ") + hipGetErrorString(e));
     return GLA_OK;
@@ -1010,8 +978,9 @@ gla_status gla_opr_apply_noalloc(gla_opr_t h, const void* x, int64_t nx, void* y
     // whose partitions do not fit together runs pair by pair
     auto bytes1 = [&](Slots s) { return ((size_t)(h->geom.w1s * s.w1) * eb + 255) & ~(size_t)255; };
     auto bytes = [&](Slots s) { return bytes1(s) + (size_t)(h->geom.w2s * s.w2) * eb; };
-    Slots have = part_slots(*h, nrhs);
-    if (bytes(have) > kScratchBytes) have = pair_slots(nrhs);
+    const gla::SlotCost cost = slot_cost(*h);
+    Slots have = gla::part_slots(cost, nrhs);
+    if (nrhs > gla::part_limit(cost) || bytes(have) > kScratchBytes) have = gla::pair_slots(nrhs);
     const size_t w1b = bytes1(have), need = bytes(have);
     if (need > kScratchBytes)
         return fail(GLA_ERR_SIZE, "the allocation-free matvec needs " + std::to_string(need) +
@@ -1150,8 +1119,8 @@ gla_status profile_seq_locked(gla_opr_t h, const void* x, void* y, int64_t nrhs,
         e = hipEventRecord(ev[(size_t)r * ne], st);
         for (int p = 0; p < gla::NPASS && e == hipSuccess; ++p) {
             e = h->dims.dtype == GLA_C64
-                    ? gla::run_pass<float>(p, G, h->tab, x, y, h->w1, h->w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(), st)
-                    : gla::run_pass<double>(p, G, h->tab, x, y, h->w1, h->w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(),
+                    ? gla::run_pass<float>(p, G, h->tab, x, y, h->ws.w1, h->ws.w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(), st)
+                    : gla::run_pass<double>(p, G, h->tab, x, y, h->ws.w1, h->ws.w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(),
                                             st);
             if (e == hipSuccess) e = hipEventRecord(ev[(size_t)r * ne + p + 1], st);
         }
@@ -1207,8 +1176,8 @@ gla_status profile_locked(gla_opr_t h, const void* x, void* y, int64_t nrhs, voi
         (void)hipEventRecord(e0, st);
         for (int r = 0; r < reps && e == hipSuccess; ++r)
             e = h->dims.dtype == GLA_C64
-                    ? gla::run_pass<float>(p, G, h->tab, x, y, h->w1, h->w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(), st)
-                    : gla::run_pass<double>(p, G, h->tab, x, y, h->w1, h->w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(),
+                    ? gla::run_pass<float>(p, G, h->tab, x, y, h->ws.w1, h->ws.w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(), st)
+                    : gla::run_pass<double>(p, G, h->tab, x, y, h->ws.w1, h->ws.w2, (int)nrhs, 1, 0, 0, 0, 0, gla::Epi(),
                                             st);
         (void)hipEventRecord(e1, st);
         if (e == hipSuccess) e = hipEventSynchronize(e1);
@@ -1320,7 +1289,7 @@ gla_status gla_batch_create(const gla_opr_t* ops, const void* const* x, void* co
         std::lock_guard<std::mutex> lk(h->mu);
         const int r = (int)(nrhs ? nrhs[i] : 1);
         hipStream_t st = ls[(size_t)lane[(size_t)i]];
-        e = matvec_all(*h, x[i], y[i], h->w1, h->w2, Slots{h->w1_slots, h->w2_slots}, r, 1, 0, 0, 0, 0, gla::Epi(), st);
+        e = matvec_all(*h, x[i], y[i], h->ws.w1, h->ws.w2, h->ws.held, r, 1, 0, 0, 0, 0, gla::Epi(), st);
     }
     for (int k = 0; k < lanes && e == hipSuccess; ++k) e = hipEventRecord(ev[(size_t)k], ls[(size_t)k]);
     for (int k = 0; k < lanes && e == hipSuccess; ++k) e = hipStreamWaitEvent(cap, ev[(size_t)k], 0);   // join
@@ -1372,8 +1341,9 @@ gla_status gla_opr_reserve(gla_opr_t h, int64_t nrhs)
 int64_t gla_opr_workspace_bytes(gla_opr_t h, int64_t nrhs)
 {
     if (!h) return -1;
-    const Slots s = part_slots(*h, nrhs);
-    return (h->geom.w1s * s.w1 + h->geom.w2s * s.w2) * (int64_t)elem_bytes(h->dims.dtype);
+    const gla::SlotCost c = slot_cost(*h);
+    const Slots s = gla::want_slots(c, nrhs);
+    return c.w1 * s.w1 + c.w2 * s.w2;
 }
 
 int64_t gla_krylov_dots_workspace(int64_t k, int64_t nv, int64_t n)

@@ -249,8 +249,10 @@ gla_status gla_opr_load(const char* path, int32_t dtype, int32_t device, gla_opr
 
 /* Grow the handle's work buffers to nrhs right-hand sides now.  An apply on
  * a stream under HIP graph capture must not allocate, so it fails with
- * GLA_ERR_ARG instead of growing them: reserve before capturing.  No
- * counterpart in the reference (its device path allocates per call). */
+ * GLA_ERR_ARG instead of growing them: reserve before capturing.  Calls with
+ * at most the largest count applied, reserved or captured so far never move
+ * the buffers; a larger one may, and then invalidates graphs captured before.
+ * No counterpart in the reference (its device path allocates per call). */
 gla_status gla_opr_reserve(gla_opr_t h, int64_t nrhs);
 
 /* ---- Recorded batches of operators ------------------------------------
@@ -271,7 +273,8 @@ gla_status gla_batch_create(const gla_opr_t* ops, const void* const* x, void* co
 gla_status gla_batch_launch(gla_batch_t b, void* stream);
 gla_status gla_batch_destroy(gla_batch_t b);
 
-/* Bytes of device work memory the handle holds for nrhs right-hand sides. */
+/* Bytes of device work memory the handle holds for nrhs right-hand sides (a
+ * partitioned operator less where so much could not be allocated). */
 int64_t gla_opr_workspace_bytes(gla_opr_t h, int64_t nrhs);
 
 /* ---- Batched Krylov-basis reductions (GMRES building blocks) ------------
