@@ -718,7 +718,9 @@ __global__ void k_idft_axis(double2* __restrict__ out, const double2* __restrict
 
 // the circulant of an exact grid L = S + T re-embedded on a grid L' >= L:
 // separations 0..T-1 at n' = n, -(S-1)..-1 at the top of L'; zero elsewhere;
-// scaled by `scale` (the inverse transform's 1 / (L1 L2 L3))
+// scaled by `scale` (the inverse transform's 1 / (L1 L2 L3)).  An axis that
+// keeps its length keeps every entry: without the one separation no pair of
+// cells has, a symmetric axis stored by half could lose its mirror relation.
 __global__ void k_reembed(double2* __restrict__ out, const double2* __restrict__ in, int L1, int L2, int L3,
                           int M1, int M2, int M3, int T1, int T2, int T3, int S1, int S2, int S3, double scale)
 {
@@ -728,7 +730,7 @@ __global__ void k_reembed(double2* __restrict__ out, const double2* __restrict__
     const int64_t q = p % Mt;
     const int c = (int)(p / Mt);
     const int m1 = (int)(q % M1), m2 = (int)((q / M1) % M2), m3 = (int)(q / ((int64_t)M1 * M2));
-    auto src = [](int m, int M, int L, int T, int S) { return m < T ? m : (m > M - S ? m - M + L : -1); };
+    auto src = [](int m, int M, int L, int T, int S) { return m < T || M == L ? m : (m > M - S ? m - M + L : -1); };
     const int n1 = src(m1, M1, L1, T1, S1), n2 = src(m2, M2, L2, T2, S2), n3 = src(m3, M3, L3, T3, S3);
     if (n1 < 0 || n2 < 0 || n3 < 0) {
         out[p] = make_double2(0, 0);

@@ -3,7 +3,7 @@ used as it is given: the longer spectrum it is re-expressed at is its own
 mirror image only if the data's self-image entries (frequency 0 and L / 2) of
 the components odd in the axis vanish, so mirror storage of G^ may not be
 assumed.  Random branches against the oracle, on self operators with every
-axis re-embedded and on the symmetric axis of an external pair."""
+axis re-embedded or some of them, and on the symmetric axis of an external pair."""
 import numpy as np
 import pytest
 
@@ -14,6 +14,7 @@ H = ((1, 32),) * 3
 CASES = {
     "self_7_9_11": ((7, 9, 11), (7, 9, 11), (0, 0, 0), (1, 1, 1)),
     "self_14_7_33": ((14, 7, 33), (14, 7, 33), (0, 0, 0), (1, 1, 1)),
+    "self_14_8_33": ((14, 8, 33), (14, 8, 33), (0, 0, 0), (1, 1, 1)),
     "external_axis_2": ((10, 7, 4), (16, 7, 8), ((1, 2), 0, (3, 4)), (0, 1, 0)),
 }
 
