@@ -21,7 +21,8 @@ length (compile-time overrides of gla_tune.hpp):
   xk     passes 1 and 5: the two parities of a row through the stages
          together or one after the other, timed on the rows grid
   gg     pass 3: the first point's G^ loads issued before the forward
-         transform or not, timed on the large cross-section
+         transform or not, or every point's ahead of the product, timed on
+         the large cross-section
   yk     passes 2 and 4: the two parities of a bundle together or in turn,
          timed on the rows grid
   rl     pass 3: the input column kept, read again or split into both
@@ -30,7 +31,7 @@ length (compile-time overrides of gla_tune.hpp):
 Operators come from all-zero Green data (the timing does not depend on the
 values), so no setup runs.  Each (part, element type, length[, class]) keeps
 its current table entry (or default) unless a candidate beats it by more than
---margin (5%): a timing grid is not every workload, and differences within
+--margin (5%); an entry that was not measured stays: a timing grid is not every workload, and differences within
 the run-to-run noise stay with the incumbent.  (A 64 x 64 x N grid for every
 length understated the pass-3 gain of a shape at 96^3 threefold against the
 cube: the cross-section matters, hence the classes.)
@@ -75,8 +76,8 @@ def candidates():
     out.append(("p0", "-DGLA_PT_F=0 -DGLA_PT_D=0", {"part": "plan", "c64": 0, "c128": 0}))
     out.append(("x1", "-DGLA_XK_F=1 -DGLA_XK_D=1", {"part": "xk", "c64": 1, "c128": 1}))
     out.append(("x2", "-DGLA_XK_F=2 -DGLA_XK_D=2", {"part": "xk", "c64": 2, "c128": 2}))
-    out.append(("g3", "-DGLA_ZGG_F=3 -DGLA_ZGG_D=3", {"part": "gg", "c64": 3, "c128": 3}))
-    out.append(("g7", "-DGLA_ZGG_F=7 -DGLA_ZGG_D=7", {"part": "gg", "c64": 7, "c128": 7}))
+    for v in (3, 7, 15):
+        out.append((f"g{v}", f"-DGLA_ZGG_F={v} -DGLA_ZGG_D={v}", {"part": "gg", "c64": v, "c128": v}))
     out.append(("y1", "-DGLA_YK_F=1 -DGLA_YK_D=1", {"part": "yk", "c64": 1, "c128": 1}))
     out.append(("y2", "-DGLA_YK_F=2 -DGLA_YK_D=2", {"part": "yk", "c64": 2, "c128": 2}))
     for v in (0, 1, 2):
@@ -168,10 +169,15 @@ def _current(src, tag, pat):
 
 
 def _decide(by, incumbent, margin):
-    """The fastest choice when it beats the incumbent by more than `margin`
-    (or the incumbent was not measured), else the incumbent."""
+    """The fastest choice when it beats the incumbent by more than `margin`,
+    else the incumbent; one that was not measured is not beaten."""
     best = min(by, key=by.get)
-    return best if incumbent not in by or by[best] < (1 - margin) * by[incumbent] else incumbent
+    return best if incumbent in by and by[best] < (1 - margin) * by[incumbent] else incumbent
+
+
+def _at(by, choice):
+    """A choice's time for the report, or that it has none."""
+    return f"{by[choice]:.1f} us" if choice in by else "not measured"
 
 
 def table(results, margin):
@@ -200,7 +206,7 @@ def table(results, margin):
             d = vals.get(n, dflt)
             c = _decide(byn[n], d, margin)
             vals[n] = c
-            lines.append(f"{dt} {part} {n}: {c} ({byn[n][c]:.1f} us {what}; current {d} {byn[n].get(d, 0):.1f})")
+            lines.append(f"{dt} {part} {n}: {c} ({_at(byn[n], c)} {what}; current {d} {_at(byn[n], d)})")
         src = _sub(src, tname, [f"            case {n}: return {v};" for n, v in sorted(vals.items()) if v != dflt])
 
     for dt, tag in (("c64", "C64"), ("c128", "C128")):
@@ -218,12 +224,12 @@ def table(results, margin):
             for n, by in zl.items():
                 d = large.get(n, ZDEFAULT[dt])
                 large[n] = _decide(by, d, margin)
-                lines.append(f"{dt} zpass large {n}: {large[n]} {by[large[n]]:.1f} us (current {d} {by.get(d, 0):.1f})")
+                lines.append(f"{dt} zpass large {n}: {large[n]} {_at(by, large[n])} (current {d} {_at(by, d)})")
             for n, by in zs.items():
                 ref = large[n]
                 small[n] = _decide(by, ref, margin)
-                lines.append(f"{dt} zpass small {n}: {small[n]} {by[small[n]]:.1f} us (large-grid shape {ref} "
-                             f"{by.get(ref, 0):.1f})")
+                lines.append(f"{dt} zpass small {n}: {small[n]} {_at(by, small[n])} (large-grid shape {ref} "
+                             f"{_at(by, ref)})")
             src = _sub(src, tag, [f"            case {n}: return {{{s[0]}, {s[1]}}};"
                                   for n, s in sorted(large.items()) if s != ZDEFAULT[dt]])
             src = _sub(src, tag + " SMALL", [f"            case {n}: return {{{s[0]}, {s[1]}}};"
@@ -245,7 +251,7 @@ def table(results, margin):
                 ex = _decide(rx[n], d[0], margin)
                 ey = _decide(ry[n], (d[1], d[2]), margin)
                 rows[n] = (ex, ey[0], ey[1])
-                lines.append(f"{dt} rows {n}: ex {ex} ({rx[n][ex]:.1f} us), ey/pxy {ey} ({ry[n][ey]:.1f} us); "
+                lines.append(f"{dt} rows {n}: ex {ex} ({_at(rx[n], ex)}), ey/pxy {ey} ({_at(ry[n], ey)}); "
                              f"current {d}")
             src = _sub(src, "ROWS " + tag, [f"            case {n}: return RShape{{{v[0]}, {v[1]}, {v[2]}}};"
                                             for n, v in sorted(rows.items()) if v != rdefault(dt, n)])

@@ -1,0 +1,46 @@
+"""The autotuner against the tables it keeps: its recorded results leave every
+entry where it is (entries they did not measure included), and each entry of
+the single-value tables is one of its candidates, so a new run can weigh it."""
+import importlib.util
+import json
+import os
+import re
+import shutil
+
+import pytest
+
+PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "gilaelectromagnetics.jl_amd")
+
+
+@pytest.fixture()
+def tune(tmp_path):
+    spec = importlib.util.spec_from_file_location("gla_tune_entries", os.path.join(PKG, "tune.py"))
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    shutil.copy(os.path.join(PKG, "csrc", "gla_tune.hpp"), tmp_path / "gla_tune.hpp")
+    mod.CSRC = str(tmp_path)
+    return mod
+
+
+def test_recorded_results_keep_the_tables(tune, tmp_path):
+    before = (tmp_path / "gla_tune.hpp").read_text()
+    tune.table(os.path.join(PKG, "tune", "shapes_mi355x.jsonl"), 0.05)
+    assert (tmp_path / "gla_tune.hpp").read_text() == before
+
+
+def test_entries_are_candidates(tune, tmp_path):
+    src = (tmp_path / "gla_tune.hpp").read_text()
+    for part, tag in (("gg", "GG"), ("xk", "XK"), ("yk", "YK"), ("rl", "RELOAD"), ("plan", "PLAN")):
+        for dt in ("c64", "c128"):
+            have = {d[dt] for _, _, d in tune.candidates() if d["part"] == part}
+            body = re.search(rf"// BEGIN TUNED {tag} {dt.upper()}\n(.*?)// END TUNED", src, flags=re.S).group(1)
+            assert {int(v) for v in re.findall(r"return (\d+);", body)} <= have, (part, dt)
+
+
+def test_a_measured_entry_can_lose(tune, tmp_path):
+    path = tmp_path / "res.jsonl"
+    path.write_text("\n".join(json.dumps({"part": "gg", "dtype": "c128", "n": 64, "choice": c,
+                                          "large_us": [0, 0, t, 0, 0]}) for c, t in ((3, 80.0), (7, 90.0), (15, 100.0))))
+    tune.table(str(path), 0.05)
+    body = re.search(r"// BEGIN TUNED GG C128\n(.*?)// END TUNED", (tmp_path / "gla_tune.hpp").read_text(), flags=re.S)
+    assert "case 64:" not in body.group(1) and "case 128: return 15;" in body.group(1)
