@@ -39,6 +39,7 @@
 //   -DGLA_YK_F=.. / -DGLA_YK_D=.. (or -DGLA_YK=.. for both)
 //   -DGLA_ZRELOAD_F=.. / -DGLA_ZRELOAD_D=..
 //   -DGLA_PT_F=.. / -DGLA_PT_D=..
+//   -DGLA_WT_F=0 (k_zpass at every length)
 // (_F: ComplexF32, _D: ComplexF64.)
 #pragma once
 
@@ -135,7 +136,8 @@ constexpr ZShape ztune(int complex_bytes, int n, bool small)
 
 // pass 3, wave form (k_zwave): threads per pencil, column groups of 64 / tp
 // columns per workgroup, waves per SIMD asked of the compiler and G^ points in
-// flight; tp 0: the length runs k_zpass.  Taken where k_zpass's plan wastes
+// flight; tp 0: the length runs k_zpass.  At the lengths listed, ztune's
+// elements per thread serve only partitioned operators (k_zpart).  Taken where k_zpass's plan wastes
 // lanes or exchanges (96 = 4 6 4 against 4 3 2 4; 160, 192): us of pass 3,
 // k_zpass / k_zwave: 16 right-hand sides of 96^3 1113 / 999, 96^3 65.3 / 63.1,
 // 160^3 458 / 370, 192^3 716 / 638; not where it does not (128^3 153 / 179,
@@ -146,14 +148,21 @@ struct WShape {
 
 constexpr WShape wtune(int complex_bytes, int n)
 {
+#if defined(GLA_WT_F) && GLA_WT_F == 0
+    (void)complex_bytes;
+    (void)n;
+#else
     if (complex_bytes == 8) {
         switch (n) {
+            // BEGIN WAVE C64
             case 96: return {8, 2, 2, 2};
             case 160: return {8, 2, 2, 2};
             case 192: return {8, 2, 2, 2};
-            default: return {0, 0, 0, 0};
+            // END WAVE C64
+            default: break;
         }
     }
+#endif
     return {0, 0, 0, 0};
 }
 

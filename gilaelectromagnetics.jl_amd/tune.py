@@ -5,13 +5,16 @@ element type and grid shape; writes the tables of csrc/gla_tune.hpp.
     python tune.py measure --out DIR > res.jsonl  # on the GPU
     python tune.py table   res.jsonl              # rewrites csrc/gla_tune.hpp
 
-Seven parts, each a set of candidate libraries that force one choice for every
+Eight parts, each a set of candidate libraries that force one choice for every
 length (compile-time overrides of gla_tune.hpp):
 
   zpass  pass 3: (elements per thread, columns per workgroup), timed on a
          large cross-section (128 x 128 x N: 256 x 256 columns) and a small
          one (64 x 64 x N: 128 x 128 columns, below ZSMALL_COLS) -- the two
-         grid classes of ztune
+         grid classes of ztune; built without the wave form, whose lengths
+         take these shapes for partitioned operators
+  wave   pass 3: the wave form at the lengths of wtune against none, timed on
+         both cross-sections; reported only (wtune is written by hand)
   rows   passes 1, 2, 4, 5: elements per thread of the axis-1 rows and the
          axis-2 columns and the axis-2 bundle width, timed on N^3 (N <= 128;
          N x N x 128 beyond: both row axes of length N)
@@ -66,8 +69,10 @@ def candidates():
     """(name, extra compile flags, description) of every candidate library."""
     out = []
     for i, (f, d) in enumerate(ZCAND):
-        out.append((f"z{i}", f"-DGLA_ZT_E_F={f[0]} -DGLA_ZT_PX_F={f[1]} -DGLA_ZT_E_D={d[0]} -DGLA_ZT_PX_D={d[1]}",
+        out.append((f"z{i}", f"-DGLA_WT_F=0 -DGLA_ZT_E_F={f[0]} -DGLA_ZT_PX_F={f[1]} -DGLA_ZT_E_D={d[0]} -DGLA_ZT_PX_D={d[1]}",
                     {"part": "zpass", "c64": f, "c128": d}))
+    out.append(("w0", "-DGLA_WT_F=0", {"part": "wave", "c64": 0, "c128": 0}))
+    out.append(("w1", "", {"part": "wave", "c64": 1, "c128": 1}))
     for i, (f, d) in enumerate(RCAND):
         out.append((f"r{i}", f"-DGLA_RT_EX_F={f[0]} -DGLA_RT_EY_F={f[1]} -DGLA_RT_PXY_F={f[2]} "
                              f"-DGLA_RT_EX_D={d[0]} -DGLA_RT_EY_D={d[1]} -DGLA_RT_PXY_D={d[2]}",
@@ -133,9 +138,9 @@ def measure_one(name, lengths):
     for n in lengths:
         for typ, dt in ((np.complex64, "c64"), (np.complex128, "c128")):
             rec = {"cand": name, "part": part, "dtype": dt, "n": n, "choice": desc[dt]}
-            if part in ("zpass", "plan", "gg", "rl"):
+            if part in ("zpass", "wave", "plan", "gg", "rl"):
                 rec["large_us"] = timed((128, 128, n), typ)
-            if part == "zpass":
+            if part in ("zpass", "wave"):
                 rec["small_us"] = timed((64, 64, n), typ)
             if part in ("rows", "plan", "xk", "yk"):
                 rec["rows_us"] = timed((n, n, min(n, 128)), typ)
@@ -208,6 +213,17 @@ def table(results, margin):
             vals[n] = c
             lines.append(f"{dt} {part} {n}: {c} ({_at(byn[n], c)} {what}; current {d} {_at(byn[n], d)})")
         src = _sub(src, tname, [f"            case {n}: return {v};" for n, v in sorted(vals.items()) if v != dflt])
+
+    # the wave form, reported where it is taken
+    wave = {}
+    for r in recs:
+        if r["part"] == "wave" and r["dtype"] == "c64":
+            wave.setdefault(r["n"], {})[r["choice"]] = r
+    wrows = re.search(r"// BEGIN WAVE C64\n(.*?)// END WAVE C64", src, flags=re.S).group(1)
+    for n in sorted(set(wave) & {int(v) for v in re.findall(r"case (\d+):", wrows)}):
+        for grid in ("large", "small"):
+            by = {c: r[grid + "_us"][2] for c, r in wave[n].items()}
+            lines.append(f"c64 wave {n} {grid}: wave form {_at(by, 1)}, without {_at(by, 0)}")
 
     for dt, tag in (("c64", "C64"), ("c128", "C128")):
         # pass 3 by grid class: the large-grid table, then small-grid entries

@@ -44,3 +44,20 @@ def test_a_measured_entry_can_lose(tune, tmp_path):
     tune.table(str(path), 0.05)
     body = re.search(r"// BEGIN TUNED GG C128\n(.*?)// END TUNED", (tmp_path / "gla_tune.hpp").read_text(), flags=re.S)
     assert "case 64:" not in body.group(1) and "case 128: return 15;" in body.group(1)
+
+
+def test_wave_lengths_are_timed_with_and_without(tune, tmp_path, capsys):
+    # at the wave form's lengths pass 3's shapes time k_zpass, so that they
+    # differ, and the wave form itself is compared and reported
+    assert all("-DGLA_WT_F=0" in flags for _, flags, d in tune.candidates() if d["part"] == "zpass")
+    assert {flags for _, flags, d in tune.candidates() if d["part"] == "wave"} == {"-DGLA_WT_F=0", ""}
+    before = (tmp_path / "gla_tune.hpp").read_text()
+    assert "GLA_WT_F == 0" in before
+    path = tmp_path / "res.jsonl"
+    path.write_text("\n".join(json.dumps({"part": "wave", "dtype": "c64", "n": n, "choice": c,
+                                          "large_us": [0, 0, t, 0, 0], "small_us": [0, 0, t / 4, 0, 0]})
+                              for n in (96, 128) for c, t in ((0, 60.0), (1, 50.0))))
+    tune.table(str(path), 0.05)
+    out = capsys.readouterr().out
+    assert "c64 wave 96 large: wave form 50.0 us, without 60.0 us" in out and "wave 128" not in out
+    assert (tmp_path / "gla_tune.hpp").read_text() == before
