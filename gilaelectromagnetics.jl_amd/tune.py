@@ -17,7 +17,9 @@ length (compile-time overrides of gla_tune.hpp):
          both cross-sections; reported only (wtune is written by hand)
   rows   passes 1, 2, 4, 5: elements per thread of the axis-1 rows and the
          axis-2 columns and the axis-2 bundle width, timed on N^3 (N <= 128;
-         N x N x 128 beyond: both row axes of length N)
+         N x N x 128 beyond: both row axes of length N); lengths up to 64 as
+         whole applies, which take the elements per thread for the plane
+         kernels there
   plan   the radix plan policy (every thread busy in every stage, against the
          fewest LDS exchanges) for all passes of a length, timed as pass 3 on
          the large cross-section plus the row passes on the rows grid
@@ -56,7 +58,9 @@ ZCAND = [((8, 16), (4, 8)), ((4, 8), (2, 8)), ((4, 16), (4, 4)), ((8, 8), (8, 4)
          ((2, 8), (4, 16))]
 ZDEFAULT = {"c64": (8, 16), "c128": (4, 8)}
 # rows: ((ex, ey, pxy) ComplexF32, (ex, ey, pxy) ComplexF64)
-RCAND = [((4, 4, 16), (4, 4, 8)), ((8, 8, 16), (8, 8, 8)), ((4, 8, 8), (4, 8, 4)), ((8, 4, 32), (8, 4, 16))]
+RCAND = [((4, 4, 16), (4, 4, 8)), ((8, 8, 16), (8, 8, 8)), ((4, 8, 8), (4, 8, 4)), ((8, 4, 32), (8, 4, 16)),
+         ((8, 4, 16), (8, 4, 8))]
+PLANES = 64   # N x N planes up to here run passes 1 + 2 and 4 + 5 as one kernel each
 
 
 def rdefault(dt, n):
@@ -115,7 +119,8 @@ def measure_one(name, lengths):
     desc = {n: d for n, _, d in candidates()}[name]
     part = desc["part"]
 
-    def timed(N, typ):
+    def timed(N, typ, whole=False):
+        """us of the five passes, or of a whole apply in turn"""
         vol = gila.GlaVol(N, (Fraction(1, 32),) * 3)
         dims = _capi.gla_dims()
         _capi.check(gila.lib().gla_opr_dims_for(ctypes.byref(vol._c()), None, ctypes.byref(dims)))
@@ -128,6 +133,16 @@ def measure_one(name, lengths):
         ms = (ctypes.c_double * 5)()
         by = (ctypes.c_int64 * 5)()
         st = torch.cuda.current_stream().cuda_stream
+        if whole:
+            ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+            for r in range(120):
+                if r == 20:
+                    ev[0].record()
+                _capi.check(gila.lib().gla_opr_apply(mem._h, ctypes.c_void_p(xd.data_ptr()), n,
+                                                     ctypes.c_void_p(yd.data_ptr()), n, 1, ctypes.c_void_p(st)))
+            ev[1].record()
+            torch.cuda.synchronize()
+            return ev[0].elapsed_time(ev[1]) * 10.0
         _capi.check(gila.lib().gla_opr_profile(mem._h, ctypes.c_void_p(xd.data_ptr()), n,
                                                ctypes.c_void_p(yd.data_ptr()), n, 1, ctypes.c_void_p(st), 10, ms,
                                                by))
@@ -144,6 +159,8 @@ def measure_one(name, lengths):
                 rec["small_us"] = timed((64, 64, n), typ)
             if part in ("rows", "plan", "xk", "yk"):
                 rec["rows_us"] = timed((n, n, min(n, 128)), typ)
+            if part == "rows" and n <= PLANES:
+                rec["apply_us"] = timed((n, n, n), typ, whole=True)
             print(json.dumps(rec), flush=True)
 
 
@@ -251,8 +268,9 @@ def table(results, margin):
             src = _sub(src, tag + " SMALL", [f"            case {n}: return {{{s[0]}, {s[1]}}};"
                                              for n, s in sorted(small.items())
                                              if s != large.get(n, ZDEFAULT[dt])])
-        # rows: axis-1 passes (1 + 5) by ex, axis-2 passes (2 + 4) by (ey, pxy)
-        rx, ry = {}, {}
+        # rows: axis-1 passes (1 + 5) by ex, axis-2 passes (2 + 4) by (ey, pxy);
+        # where planes run, the whole entry by the apply
+        rx, ry, ra = {}, {}, {}
         for r in recs:
             if r["part"] != "rows" or r["dtype"] != dt:
                 continue
@@ -260,10 +278,16 @@ def table(results, margin):
             t = r["rows_us"]
             rx.setdefault(r["n"], {})[ex] = min(t[0] + t[4], rx.get(r["n"], {}).get(ex, 1e30))
             ry.setdefault(r["n"], {})[(ey, pxy)] = t[1] + t[3]
+            if "apply_us" in r:
+                ra.setdefault(r["n"], {})[(ex, ey, pxy)] = r["apply_us"]
         if rx:
             rows = dict(_current(src, "ROWS " + tag, rpat))
             for n in sorted(rx):
                 d = rows.get(n, rdefault(dt, n))
+                if n in ra:
+                    rows[n] = _decide(ra[n], d, margin)
+                    lines.append(f"{dt} rows {n}: {rows[n]} {_at(ra[n], rows[n])} an apply (current {d} {_at(ra[n], d)})")
+                    continue
                 ex = _decide(rx[n], d[0], margin)
                 ey = _decide(ry[n], (d[1], d[2]), margin)
                 rows[n] = (ex, ey[0], ey[1])

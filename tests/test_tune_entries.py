@@ -61,3 +61,24 @@ def test_wave_lengths_are_timed_with_and_without(tune, tmp_path, capsys):
     out = capsys.readouterr().out
     assert "c64 wave 96 large: wave form 50.0 us, without 60.0 us" in out and "wave 128" not in out
     assert (tmp_path / "gla_tune.hpp").read_text() == before
+
+
+def test_rows_of_plane_lengths_by_the_apply(tune, tmp_path):
+    # 16: the plane kernels' apply decides, whatever the five separate passes
+    # say; 80: the passes decide; entries that were set are candidates
+    recs = []
+    for (ex, ey, pxy), t in (((4, 4, 16), 30.0), ((8, 8, 16), 20.0), ((8, 4, 16), 25.0)):
+        recs.append({"part": "rows", "dtype": "c64", "n": 16, "choice": [ex, ey, pxy], "apply_us": t,
+                     "rows_us": [40 - t, 40 - t, 0, 0, 0]})
+        recs.append({"part": "rows", "dtype": "c64", "n": 80, "choice": [ex, ey, pxy],
+                     "rows_us": [40 - t, 40 - t, 0, 0, 0]})
+    path = tmp_path / "res.jsonl"
+    path.write_text("\n".join(map(json.dumps, recs)))
+    tune.table(str(path), 0.05)
+    src = (tmp_path / "gla_tune.hpp").read_text()
+    body = re.search(r"// BEGIN TUNED ROWS C64\n(.*?)// END TUNED", src, flags=re.S).group(1)
+    assert "case 16: return RShape{8, 8, 16};" in body and "case 80:" not in body
+    for k, dt in enumerate(("C64", "C128")):
+        body = re.search(rf"// BEGIN TUNED ROWS {dt}\n(.*?)// END TUNED", src, flags=re.S).group(1)
+        small = [tuple(map(int, v)) for v in re.findall(r"case (\d+): return RShape\{(\d+), (\d+), (\d+)\}", body)]
+        assert {v[1:] for v in small if v[0] <= 64} <= {c[k] for c in tune.RCAND}
