@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <complex>
@@ -342,27 +343,64 @@ struct AxisStore {
     bool sym;
 };
 
+// What is known of the branches along an embedded axis on which source and
+// target coincide: their own mirror images, not, or to be checked.
+enum class Mirror { yes, no, check };
+using Mirrors = std::array<Mirror, 3>;
+constexpr Mirrors kMade{Mirror::yes, Mirror::yes, Mirror::yes};
+constexpr Mirrors kUnknown{Mirror::check, Mirror::check, Mirror::check};
+
+// the off-diagonal components that involve axis a, which are odd along it
+constexpr int kOdd[3][2] = {{3, 4}, {3, 5}, {4, 5}};
+
+// the largest part of any entry, and what FP64 transforms leave of a zero
+// beside it: 32 eps of it (5e-16 of it measured on re-embedded data, 6e-15 on
+// branches from face integrals)
+double fp64_noise(const std::vector<std::complex<double>>& fur)
+{
+    double top = 0;
+    for (const auto& v : fur) top = std::max(top, std::max(std::fabs(v.real()), std::fabs(v.imag())));
+    return 0x1p-47 * top;
+}
+
+// Whether branches stored by half on axis a (layout d, of which the rest
+// follows by mirroring) are still their own mirror images after re-embedding
+// on a longer length: the circulant of an odd component is odd, and stays so,
+// if its self-image entries (frequency 0 and L / 2) vanish.
+bool stays_mirrored(const gla_dims& d, const std::vector<std::complex<double>>& fur, int a)
+{
+    const int64_t U[3] = {d.fur_ext[0], d.fur_ext[1], d.fur_ext[2]};
+    const int64_t Ut = U[0] * U[1] * U[2], st = a == 0 ? 1 : a == 1 ? U[0] : U[0] * U[1];
+    const double lim = fp64_noise(fur);
+    for (int b = 0; b < 8; ++b)
+        for (int c : kOdd[a])
+            for (int64_t m : {(int64_t)0, d.brn[a]}) {
+                const int p = (b >> (2 - a)) & 1;
+                if ((m & 1) != p) continue;
+                const std::complex<double>* const f = &fur[(size_t)((b * 6 + c) * Ut)] + (m - p) / 2 * st;
+                for (int64_t lo = 0; lo < Ut; lo += st * U[a])
+                    for (int64_t i = lo; i < lo + st; ++i)
+                        if (std::fabs(f[i].real()) > lim || std::fabs(f[i].imag()) > lim) return false;
+            }
+    return true;
+}
+
 // Whether the branches are their own mirror images along axis a, F(L - m) =
-// s F(m) with s = -1 for the off-diagonal components that involve the axis
-// (the relation of a self axis), up to rounding: of the stored entries (two
+// s F(m) with s = -1 for the odd components (the relation of a self axis), up
+// to rounding: of the stored entries (two
 // ComplexF32 neighbours, `rel` of the entry) and of the FP64 transforms that
-// made them (32 eps of the largest entry; 5e-16 of it measured on re-embedded
-// data, 6e-15 on branches from face integrals).  A looser bound would lose
-// components far below the largest entry.
+// made them.  A looser bound would lose components far below the largest entry.
 bool mirrored(const gla_dims& d, const std::vector<std::complex<double>>& fur, int a)
 {
     const int64_t U[3] = {d.fur_ext[0], d.fur_ext[1], d.fur_ext[2]};
     const int64_t Ut = U[0] * U[1] * U[2], B = U[a];
     const int64_t st = a == 0 ? 1 : a == 1 ? U[0] : U[0] * U[1];
-    double top = 0;
-    for (const auto& v : fur) top = std::max(top, std::max(std::fabs(v.real()), std::fabs(v.imag())));
-    const double lim = 0x1p-47 * top, rel = d.dtype == GLA_C64 ? 0x1p-22 : 0.0;
+    const double lim = fp64_noise(fur), rel = d.dtype == GLA_C64 ? 0x1p-22 : 0.0;
     auto differ = [=](double u, double v) { return std::fabs(v - u) > lim + rel * std::fabs(u); };
-    static const int odd[3][2] = {{3, 4}, {3, 5}, {4, 5}};
     for (int b = 0; b < 8; ++b)
         for (int c = 0; c < 6; ++c) {
             const std::complex<double>* const f = &fur[(size_t)((b * 6 + c) * Ut)];
-            const double s = (c == odd[a][0] || c == odd[a][1]) ? -1.0 : 1.0;
+            const double s = (c == kOdd[a][0] || c == kOdd[a][1]) ? -1.0 : 1.0;
             const int p = (b >> (2 - a)) & 1;
             for (int64_t lo = 0; lo < Ut; lo += st * B)
                 for (int64_t k = 0; 2 * k <= B; ++k) {
@@ -381,7 +419,7 @@ bool mirrored(const gla_dims& d, const std::vector<std::complex<double>>& fur, i
 // symmetry, so pass 3 reads half the G^ per such axis (self 100x60x44 on
 // (128,64,48), ComplexF32: 151 -> 21 MB of G^, pass 3 37 -> 20 us, the call
 // 110 -> 92 us).  Data handed in or read from a file are checked, not trusted.
-AxisStore axis_store(const gla_opr_s& h, const std::vector<std::complex<double>>& fur, int a, bool made)
+AxisStore axis_store(const gla_opr_s& h, const std::vector<std::complex<double>>& fur, int a, Mirror known)
 {
     const gla_dims& d = h.dims;
     if (d.sym[a]) return AxisStore{(int)d.fur_ext[a], d.fur_ext[a] != d.brn[a]};
@@ -389,18 +427,18 @@ AxisStore axis_store(const gla_opr_s& h, const std::vector<std::complex<double>>
                       h.trg.org_num[a] * h.src.org_den[a] == h.src.org_num[a] * h.trg.org_den[a];
     const int B = (int)d.dev_brn[a];
     const bool half = same && d.dev_brn[a] != d.brn[a] && n_src_part(d) * n_trg_part(d) == 1 && B > 2 &&
-                      (made || mirrored(d, fur, a));
+                      (known == Mirror::yes || (known == Mirror::check && mirrored(d, fur, a)));
     return half ? AxisStore{B / 2 + 1, true} : AxisStore{(int)d.fur_ext[a], false};
 }
 
 template <typename R>
-gla_status upload(gla_opr_t h, const std::vector<std::complex<double>>& furd, bool made)
+gla_status upload(gla_opr_t h, const std::vector<std::complex<double>>& furd, const Mirrors& known)
 {
     using C = std::complex<R>;
     const gla_dims& d = h->dims;
     const int64_t F0 = d.fur_ext[0], F1 = d.fur_ext[1], Ft = F0 * F1 * d.fur_ext[2];
     AxisStore as[3];
-    for (int a = 0; a < 3; ++a) as[a] = axis_store(*h, furd, a, made);
+    for (int a = 0; a < 3; ++a) as[a] = axis_store(*h, furd, a, known[a]);
     const int64_t U0 = as[0].U, U1 = as[1].U, U2 = as[2].U, Ut = U0 * U1 * U2;
     const int64_t P = n_src_part(d) * n_trg_part(d);
     const double scale = 1.0 / (double)(8 * d.dev_brn[0] * d.dev_brn[1] * d.dev_brn[2]);
@@ -629,7 +667,7 @@ bool finite_all(const T* p, int64_t n)
 
 namespace {
 gla_status create_common(const gla_opts* opts, const gla_vol* trg, const gla_vol* src, gla_dims d, const void* fur,
-                         int32_t fur_dtype, int64_t fur_len, bool made, gla_opr_t* out);
+                         int32_t fur_dtype, int64_t fur_len, const Mirrors& known, gla_opr_t* out);
 }
 
 extern "C" {
@@ -652,7 +690,7 @@ gla_status gla_opr_create_from_fur(const gla_opts* opts, const gla_vol* trg, con
     if ((s = dims_impl(&t2, sp, DIMS_EXACT, &d))) return s;
     bool same = true;
     for (int a = 0; a < 3; ++a) same = same && d.dev_brn[a] == ref.brn[a];
-    if (same) return create_common(opts, &t2, sp, d, fur, fur_dtype, fur_len, false, out);
+    if (same) return create_common(opts, &t2, sp, d, fur, fur_dtype, fur_len, kUnknown, out);
     // a branch length without a compiled transform: the data is re-expressed
     // at the next fast length (gla::refur) in FP64
     const int64_t Ut = ref.fur_ext[0] * ref.fur_ext[1] * ref.fur_ext[2];
@@ -672,20 +710,19 @@ gla_status gla_opr_create_from_fur(const gla_opts* opts, const gla_vol* trg, con
         DevGuard g(opts->device);
         if ((s = gla::refur(ref, d, furd, re, err))) return fail(s, err);
     }
-    return create_common(opts, &t2, sp, d, re.data(), GLA_C128, (int64_t)re.size(), false, out);
+    Mirrors known;
+    for (int a = 0; a < 3; ++a) known[a] = ref.sym[a] && stays_mirrored(ref, furd, a) ? Mirror::yes : Mirror::no;
+    return create_common(opts, &t2, sp, d, re.data(), GLA_C128, (int64_t)re.size(), known, out);
 }
 
 }  // extern "C"
 
 namespace {
 
-// made: the branches come from this library's own setup, so an embedded
-// axis's mirror symmetry needs no check.  Branches handed in do, re-embedded
-// ones too: the longer spectrum is its own mirror image only if their
-// self-image entries (frequency 0 and L / 2) of the components odd in the
-// axis vanish.
+// known: of an embedded axis's mirror symmetry -- kMade for branches of this
+// library's own setup
 gla_status create_common(const gla_opts* opts, const gla_vol* trg, const gla_vol* src, gla_dims d, const void* fur,
-                         int32_t fur_dtype, int64_t fur_len, bool made, gla_opr_t* out)
+                         int32_t fur_dtype, int64_t fur_len, const Mirrors& known, gla_opr_t* out)
 {
     gla_status s;
     const int64_t Ut = d.fur_ext[0] * d.fur_ext[1] * d.fur_ext[2];
@@ -716,7 +753,7 @@ gla_status create_common(const gla_opts* opts, const gla_vol* trg, const gla_vol
     fill_geom(h.get());
     {
         DevGuard g(opts->device);
-        s = opts->dtype == GLA_C64 ? upload<float>(h.get(), furd, made) : upload<double>(h.get(), furd, made);
+        s = opts->dtype == GLA_C64 ? upload<float>(h.get(), furd, known) : upload<double>(h.get(), furd, known);
         if (s) return s;
     }
     // host copy in the operator's element type, rounded as the reference's
@@ -757,7 +794,7 @@ gla_status gla_opr_create(const gla_opts* opts, const gla_vol* trg, const gla_vo
     std::string err;
     s = gla::setup_fur(*opts, t2, sp ? s2 : t2, d, fur, err);
     if (s) return fail(s, err);
-    return create_common(opts, &t2, sp, d, fur.data(), GLA_C128, (int64_t)fur.size(), true, out);
+    return create_common(opts, &t2, sp, d, fur.data(), GLA_C128, (int64_t)fur.size(), kMade, out);
 }
 
 gla_status gla_opr_export_fur(gla_opr_t h, void* buf, int64_t len)
@@ -929,7 +966,7 @@ gla_status gla_opr_load(const char* path, int32_t dtype, int32_t device, gla_opr
     if (o.dtype != GLA_C64 && o.dtype != GLA_C128) return fail(GLA_ERR_TYPE, "dtype must be 0, GLA_C64 or GLA_C128");
     gla_status s = gla_init(device);
     if (s) return s;
-    return create_common(&o, &hd.trg, sp, d, pay.data(), hd.dtype, (int64_t)want, false, out);
+    return create_common(&o, &hd.trg, sp, d, pay.data(), hd.dtype, (int64_t)want, kUnknown, out);
 }
 
 gla_status gla_opr_adjoint(gla_opr_t h, gla_opr_t* out)
