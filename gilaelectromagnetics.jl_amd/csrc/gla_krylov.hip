@@ -49,8 +49,8 @@ struct alignas(sizeof(cpx<R>) * VW) vec {
 // than this follows, in the update, whose reads are a step's last, from twice
 // this on -- so that the rest of it, w and the matvec's planes stay.
 // 8 right-hand sides, 16 vectors of 3 x 64 x 64 x 48 ComplexF32 elements: the
-// products 117 -> 98 us, an Arnoldi step 490 -> 470; 2 x 20 vectors of
-// 6291456 ComplexF64: both 1627 -> 1500.  The update of half that basis, 302
+// products 117 -> 98 us back to back, an Arnoldi step 490 -> 470; 2 x 20
+// vectors of 6291456 ComplexF64: both 1627 -> 1500.  The update of half that basis, 302
 // MB, with the hint 66 -> 68, and products and update in turn 115 -> 125.
 constexpr int64_t KEEP_BYTES = 192 << 20;
 
@@ -120,10 +120,12 @@ __device__ __forceinline__ void dots_count(int count, const cpx<R>* __restrict__
 // Block products of one chunk.  part layout: [r][slot][chunk]; slots 0..nv-1
 // the dots, slot nv the squared norm of w (when requested).  Bound by HBM:
 // each right-hand side's basis is read once (8 right-hand sides, 16 vectors
-// of 3 x 64 x 64 x 48 ComplexF32 elements, 640 MB: 98 us with its sums, 6.1
-// TB/s, as fast as a bare read of the basis).  Before, with 8 vectors a
-// sweep, 8-byte loads, one wave sum per value and 4096-element chunks, it
-// took 129 us, and 8 x 98304 elements 34 us (now 21).
+// of 3 x 64 x 64 x 48 ComplexF32 elements, 640 MB: 97 to 98 us with its sums
+// back to back, where the last-level cache still holds part of the basis; 112
+// to 114 us, 5.6 TB/s, and 5 for the sums inside an Arnoldi step, after the
+// matvec's planes went through that cache).  Before, with 8 vectors a sweep,
+// 8-byte loads, one wave sum per value and 4096-element chunks, it took 129
+// us back to back, and 8 x 98304 elements 34 us (now 21).
 template <typename R, int VW, bool LARGE>
 __global__ __launch_bounds__(KT) void k_dots(const cpx<R>* __restrict__ V, int64_t vr, int64_t vv,
                                              const cpx<R>* __restrict__ w, int64_t wr, int64_t n, int nv,

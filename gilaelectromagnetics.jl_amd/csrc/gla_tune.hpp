@@ -137,11 +137,12 @@ constexpr ZShape ztune(int complex_bytes, int n, bool small)
 // pass 3, wave form (k_zwave): threads per pencil, column groups of 64 / tp
 // columns per workgroup, waves per SIMD asked of the compiler and G^ points in
 // flight; tp 0: the length runs k_zpass.  At the lengths listed, ztune's
-// elements per thread serve only partitioned operators (k_zpart).  Taken where k_zpass's plan wastes
-// lanes or exchanges (96 = 4 6 4 against 4 3 2 4; 160, 192): us of pass 3,
-// k_zpass / k_zwave: 16 right-hand sides of 96^3 1113 / 999, 96^3 65.3 / 63.1,
-// 160^3 458 / 370, 192^3 716 / 638; not where it does not (128^3 153 / 179,
-// 64^3 22.2 / 21.4, 80^3 41.5 / 52.2, 96^3 ComplexF64 140 / 150).
+// elements per thread serve only partitioned operators (k_zpart).  Taken where
+// k_zpass's plan wastes lanes or exchanges (96 = 6 4 4 against 4 3 2 4; 160,
+// 192): us of pass 3, k_zpass / k_zwave: 16 right-hand sides of 96^3 1113 /
+// 999, 96^3 65.3 / 63.1, 160^3 458 / 370, 192^3 716 / 638; not where it does
+// not (128^3 153 / 179, 80^3 41.5 / 52.2, 96^3 ComplexF64 140 / 150), nor at
+// 64 (64^3 22.2 / 21.4), for less than the tables' margin of 5%.
 struct WShape {
     int tp, ng, minw, gd;
 };

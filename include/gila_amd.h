@@ -222,12 +222,13 @@ gla_status gla_opr_profile(gla_opr_t h, const void* x, int64_t nx, void* y, int6
                            int32_t reps, double* ms, int64_t* bytes);
 
 /* The same figures measured inside the real sequence: `reps` matvecs of the
- * five passes, issued as gla_opr_apply issues them (which runs passes 0 and 1,
- * and 3 and 4, of planes up to 64 x 64 branch points as one kernel each; here
- * they are timed apart), with an event at every pass boundary; ms[p] is pass p's average duration between its boundary events,
- * bytes[p] its algorithmic HBM bytes and *total_ms the average duration of
- * one whole matvec over the run.  Synchronizes; y holds a valid matvec on
- * return.  No counterpart in the reference; for benchmarks. */
+ * five passes in turn, with an event at every pass boundary; ms[p] is pass p's
+ * average duration between its boundary events, bytes[p] its algorithmic HBM
+ * bytes and *total_ms the average duration of one whole matvec of the run.
+ * gla_opr_apply runs passes 0 and 1, and 3 and 4, of planes up to 64 x 64
+ * branch points as one kernel each, which is faster than the two apart: time
+ * such an apply by two events around it.  Synchronizes; y holds a valid matvec
+ * on return.  No counterpart in the reference; for benchmarks. */
 gla_status gla_opr_profile_seq(gla_opr_t h, const void* x, int64_t nx, void* y, int64_t ny, int64_t nrhs,
                                void* stream, int32_t reps, double* ms, int64_t* bytes, double* total_ms);
 
